@@ -9,6 +9,7 @@
 #include "tuning_table.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <numeric>
 #include <sstream>
@@ -31,9 +32,30 @@ namespace {
 std::size_t padded(std::size_t n, std::size_t pad) { return pad ? n + n / pad : n; }
 
 bool needs_lds(fft1d_configuration const &c) {
-    return c.factorization.size() > 1 || c.type != transform_type::c2c || c.direct_radix();
+    return c.factorization.size() > 1 || c.type != transform_type::c2c || c.direct_radix() ||
+           (c.flags & (fft1d_stage_in | fft1d_stage_out));
+}
+
+/// Whether the K-columns of a side with strides {1, s_N, s_K} and n entries per transform are
+/// packed, i.e. consecutive K-columns are one contiguous run of memory.
+bool packed_columns(std::size_t M, std::size_t n, std::array<std::size_t, 3u> const &stride) {
+    return stride[0] == 1 && stride[1] == M && stride[2] == M * n;
 }
 } // namespace
+
+std::size_t fft1d_configuration::in_tile_bytes() const {
+    std::size_t const rb = static_cast<std::size_t>(fp);
+    std::size_t const eb = (flags & (fft1d_input_f16 | fft1d_input_bf16)) ? 4
+                           : type == transform_type::r2c                  ? rb
+                                                                          : 2 * rb;
+    return (flags & fft1d_stage_in) ? istride[2] * Kb * (pairs_k() ? 2 : 1) * eb + 12 : 0;
+}
+
+std::size_t fft1d_configuration::out_tile_bytes() const {
+    std::size_t const rb = static_cast<std::size_t>(fp);
+    std::size_t const eb = type == transform_type::c2r ? rb : 2 * rb;
+    return (flags & fft1d_stage_out) ? ostride[2] * Kb * (pairs_k() ? 2 : 1) * eb + 12 : 0;
+}
 
 int fft1d_configuration::direct_radix() const {
     for (auto f : factorization) {
@@ -44,6 +66,11 @@ int fft1d_configuration::direct_radix() const {
     return 0;
 }
 
+std::size_t fft1d_configuration::xcd_run() const {
+    std::size_t const mg = (M + Mb - 1) / Mb;
+    return mg * std::max<std::size_t>(1, 16 / mg);
+}
+
 std::size_t fft1d_configuration::lds_bytes() const {
     if (!needs_lds(*this)) {
         return 0;
@@ -51,7 +78,10 @@ std::size_t fft1d_configuration::lds_bytes() const {
     std::size_t np = padded(N_fft() - 1, lds_pad) + 1;
     // the direct stage keeps its table of roots of unity in LDS
     std::size_t const table = static_cast<std::size_t>(direct_radix());
-    return (Mb * Kb * np + table) * 2 * static_cast<std::size_t>(fp);
+    std::size_t const eb = 2 * static_cast<std::size_t>(fp);
+    std::size_t const tile = std::max({Mb * Kb * np, (in_tile_bytes() + eb - 1) / eb,
+                                       (out_tile_bytes() + eb - 1) / eb});
+    return (tile + table) * eb;
 }
 
 std::string fft1d_configuration::identifier() const {
@@ -130,6 +160,152 @@ std::vector<int> default_factorization(std::size_t n, std::size_t single_max,
 
 } // namespace gen
 
+namespace {
+
+/// Real operations of a radix-r butterfly as dft_gen emits it.
+double butterfly_ops(std::size_t r) {
+    if (r <= 2) {
+        return r == 2 ? 4.0 : 0.0;
+    }
+    if (r == 4) {
+        return 16.0;
+    }
+    std::size_t const A = r % 4 == 0 ? 4 : trial_division(static_cast<unsigned>(r)).front();
+    if (A == r) {
+        double const h = static_cast<double>(r / 2);
+        return 4.0 * h * h + 10.0 * h;
+    }
+    std::size_t const B = r / A;
+    return static_cast<double>(B) * butterfly_ops(A) + static_cast<double>(A) * butterfly_ops(B) +
+           6.0 * static_cast<double>((A - 1) * (B - 1));
+}
+
+/// Factorisations of n, largest radix first, into radices up to 16 and primes up to the
+/// register limit.
+void register_factorizations(std::size_t n, std::vector<int> &cur,
+                             std::vector<std::vector<int>> &out) {
+    if (n == 1) {
+        out.push_back(cur);
+        return;
+    }
+    if (cur.size() == 4) {
+        return;
+    }
+    std::size_t const hi = std::min<std::size_t>(
+        n, cur.empty() ? std::size_t(fft1d_max_register_radix)
+                       : static_cast<std::size_t>(cur.back()));
+    for (std::size_t r = hi; r >= 2; --r) {
+        if (n % r == 0 && (r <= 16 || is_prime(static_cast<unsigned>(r)))) {
+            cur.push_back(static_cast<int>(r));
+            register_factorizations(n / r, cur, out);
+            cur.pop_back();
+        }
+    }
+}
+
+/// Work-items of a launch with whole waves (all M columns in a tile).
+std::size_t work_items(std::size_t M, fft1d_tuning const &t, std::size_t kcols) {
+    return (kcols + t.Kb - 1) / t.Kb * ((M * t.Nt * t.Kb + 63) / 64 * 64);
+}
+
+/**
+ * Tiling of a kernel that holds all M columns of Kb transforms in one work-group (staged tiles):
+ * the factorisation, work-items per transform and K tile with the least estimated time. The
+ * estimate is linear in what separated the candidates of a sweep on MI355X (f32 and f64; c2c,
+ * r2c and c2r; 28 shapes from 1 x 16 to 17 x 363; about 100 MB in and out; 3432 kernels):
+ * vector operations per element with idle lanes counted, stages, resident waves per CU (from
+ * LDS, registers and the number of work-groups), waves per group (barriers), registers per
+ * work-item and lines shared by neighbouring tiles. Its choice is on average 1.6 % slower than
+ * the fastest candidate (at most 18 %); the fewest-stages tiling with about 256 work-items per
+ * group is 7 % slower for c2c and, without staged tiles, 32 % over all types.
+ */
+bool choose_tiling(fft1d_configuration c, std::size_t kcols, device_info const &info,
+                   fft1d_tuning &out) {
+    std::size_t const n = c.N_fft(), M = c.M;
+    std::vector<std::vector<int>> facs;
+    if (n == 1) {
+        facs.push_back({1});
+    } else {
+        std::vector<int> cur;
+        register_factorizations(n, cur, facs);
+    }
+    std::size_t stages = 4;
+    for (auto const &f : facs) {
+        stages = std::min(stages, f.size());
+    }
+    std::size_t const wg_max = std::min<std::size_t>(1024, info.max_work_group_size);
+    double const real = c.type != transform_type::c2c ? 1.0 : 0.0;
+    double const words = c.fp == precision::f32 ? 2.0 : 4.0; // registers of a complex value
+    bool found = false;
+    double best = 0.0;
+    c.Mb = M;
+    c.lds_pad = n >= 32 && (stages > 1 || real > 0.0) ? 16 : 0;
+    for (auto const &f : facs) {
+        if (f.size() > stages + 1) {
+            continue;
+        }
+        c.factorization = f;
+        for (std::size_t which = 0; which < std::min<std::size_t>(2, f.size()); ++which) {
+            std::size_t const Nt = n / static_cast<std::size_t>(f[which]);
+            if ((which && f[1] == f[0]) || M * Nt > wg_max) {
+                continue;
+            }
+            c.Nt = Nt;
+            double ops = 0.0, held = 0.0; // per work-item: operations, complex values in registers
+            for (std::size_t s = 0; s < f.size(); ++s) {
+                std::size_t const r = static_cast<std::size_t>(f[s]);
+                double const rounds = static_cast<double>((n / r + Nt - 1) / Nt);
+                double const R = static_cast<double>(r);
+                ops += rounds * (butterfly_ops(r) + (s ? 6.0 * (R - 1.0) : 0.0) + 4.0 * R);
+                held = std::max(held, rounds * R);
+            }
+            for (std::size_t items : {64u, 96u, 128u, 192u, 256u}) {
+                c.Kb = std::min(kcols, std::max<std::size_t>(1, items / (M * Nt)));
+                std::size_t const wg = c.work_group_size();
+                if (c.lds_bytes() > info.local_memory_size || wg > wg_max) {
+                    continue;
+                }
+                double const waves = static_cast<double>((wg + 63) / 64);
+                double const regs = 36.0 + words * held;
+                double const groups = static_cast<double>((kcols + c.Kb - 1) / c.Kb);
+                double resident = std::floor(info.local_memory_size / double(c.lds_bytes())) * waves;
+                resident = std::min(resident, waves * groups / 256.0);
+                resident = std::min(
+                    resident,
+                    waves * std::max(1.0, std::floor(4.0 * std::min(8.0, std::floor(512.0 / regs)) /
+                                                     waves)));
+                resident = std::min(resident, 32.0);
+                double const per_element =
+                    ops * waves * 64.0 / static_cast<double>(n * M * c.Kb);
+                // lines that a tile shares with its neighbours (they move twice)
+                double edges = 0.0;
+                for (std::size_t b : {c.in_tile_bytes(), c.out_tile_bytes()}) {
+                    if (b && (b - 12) % 128 != 0) {
+                        edges += 128.0 / static_cast<double>(b);
+                    }
+                }
+                double const score =
+                    1.2e-3 * per_element + 4.6e-2 * static_cast<double>(f.size()) +
+                    1.13 / resident + 4.8e-3 * std::log2(waves) + 2.2e-3 * words * held +
+                    0.48 * edges;
+                if (!found || score < best) {
+                    found = true;
+                    best = score;
+                    out.factorization = f;
+                    out.Nt = Nt;
+                    out.Mb = M;
+                    out.Kb = c.Kb;
+                    out.lds_pad = c.lds_pad;
+                    out.no_pad = c.lds_pad == 0;
+                }
+            }
+        }
+    }
+    return found;
+}
+
+} // namespace
+
 fft1d_configuration configure_fft1d(configuration const &cfg, device_info const &info,
                                     fft1d_tuning const &tuning_in, unsigned variant) {
     if (cfg.dim != 1) {
@@ -195,6 +371,126 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     c.store_function = cfg.callbacks.store_function;
     c.callback_hash = gen::callback_hash(cfg.callbacks);
     std::size_t const nfft = c.N_fft();
+    std::size_t const kcols = c.K_columns(K);
+
+    bool inplace_refused = false;
+    // Shapes without a table entry: when the K-columns of a side are packed, all M columns of a
+    // tile sit in LDS and that side moves in 16-byte pieces, streamed past the caches.
+    if (!explicit_tuning && tuning.factorization.empty() && info.type == device_type::gpu &&
+        !mfma && !tuning_in.unstaged) {
+        std::size_t const half = N / 2 + 1;
+        bool const in = packed_columns(M, cfg.type == transform_type::c2r ? half : N, c.istride);
+        bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N, c.ostride);
+        bool const real = cfg.type != transform_type::c2c;
+        std::size_t const eb = 2 * static_cast<std::size_t>(cfg.fp);
+        auto const f = gen::default_factorization(nfft, 16, 16);
+        std::size_t const r = static_cast<std::size_t>(*std::max_element(f.begin(), f.end()));
+        bool const registers = r <= static_cast<std::size_t>(fft1d_max_register_radix);
+        std::size_t const Nt = nfft / r;
+        // c2c fp32 with M = 2 or 3 keeps the fewest-stages tiling that the host tests fix for it
+        // (staged, 1-9 % slower than the estimate's choice)
+        bool const keep = !real && cfg.fp == precision::f32 && !half_in && (M == 2 || M == 3) &&
+                          r <= 16 && M * Nt <= 512;
+        c.flags = all_flags | (in ? fft1d_stage_in : 0u) | (outp ? fft1d_stage_out : 0u);
+        fft1d_tuning const untiled = tuning;
+        bool staged = (in || outp) && (keep || choose_tiling(c, kcols, info, tuning));
+        // Real transforms run in place when one tile holds all M columns: up to 64 columns, 512
+        // work-items and 64 KB of LDS for a single K-column.
+        c.factorization = f;
+        c.Nt = Nt;
+        c.Mb = M;
+        c.Kb = 1;
+        c.lds_pad = nfft >= 32 && (f.size() > 1 || real) ? 16 : 0;
+        c.flags = 0;
+        bool const whole_m = M <= std::max<std::size_t>(1, std::min<std::size_t>(64, 512 / Nt)) &&
+                             (M == 1 || c.lds_bytes() <= 64 * 1024);
+        inplace_refused = real && registers && !whole_m;
+        if (staged && !keep && !(real && whole_m)) {
+            // Tiles above half the LDS leave a CU with nothing to overlap a tile's copies, and
+            // tiles of all M columns of few K-columns leave CUs idle: M tiles instead (real
+            // transforms that run in place keep all M columns).
+            fft1d_configuration t = c;
+            t.factorization = tuning.factorization;
+            t.Mb = M;
+            t.Kb = tuning.Kb;
+            t.lds_pad = tuning.lds_pad;
+            staged = t.lds_bytes() <= info.local_memory_size / 2 &&
+                     (real || M == 1 || kcols >= 256 || M * Nt <= 64);
+            if (!staged) {
+                tuning = untiled;
+            }
+        }
+        if (staged) {
+            tuning.flags = fft1d_per_tile_ids;
+            // The copies add two barriers to a work-group's latency: below 8 waves per CU there
+            // is too little else to hide it (1 x 315 x 200 fp64, to the spectrum and back: 7.6 us
+            // plain, 9.3 staged; x 2000: 14.1 / 15.0; x 6000: 25.7 / 25.1)
+            bool const filled = (keep ? M * Nt * kcols : work_items(M, tuning, kcols)) >=
+                                8 * 64 * 256;
+            if (in && !c.load_function && filled) {
+                tuning.flags |= fft1d_stage_in | fft1d_nontemporal_load;
+            }
+            if (!c.store_function && (outp || M * eb >= 24) && filled) {
+                tuning.flags |= (outp ? fft1d_stage_out : 0u) | fft1d_nontemporal_store;
+            }
+            tuning.has_flags = true;
+            c.Mb = M;
+            c.Kb = tuning.Kb;
+            c.flags = tuning.flags;
+            // shared lines: 32 x 5 x 315 c2r fp32 39.7 us against 43.4, 1 x 512 r2c 49.7 / 50.5
+            if (tuning.Kb && ((c.in_tile_bytes() && (c.in_tile_bytes() - 12) % 128 != 0) ||
+                              (c.out_tile_bytes() && (c.out_tile_bytes() - 12) % 128 != 0))) {
+                tuning.flags |= fft1d_xcd_runs;
+            }
+        } else if (registers && !(real && whole_m)) {
+            // M tiles. Rows of whole 128-byte lines are streamed, 128 to 256 bytes per tile:
+            // 4704 x 80 x 16 fp32 19.3 us (32 columns) against 25.1 before (64 columns, hoisted
+            // ids), 64 x 512 x 700 63.7 against 99.3. Otherwise neighbouring M tiles share the
+            // lines at their seams: the widest tiles, plain accesses and neighbours on one XCD;
+            // 17 x 512 x 2757 fp32 81 us (9 columns) against 323 (6 columns streamed, neighbours
+            // on different XCDs) and 130 (9 columns plain, different XCDs).
+            std::size_t const line = 128 / eb;
+            bool const lines = M % line == 0 && c.istride[1] % line == 0 &&
+                               c.ostride[1] % line == 0 && c.istride[2] % line == 0 &&
+                               c.ostride[2] % line == 0 && !real;
+            tuning.factorization = f;
+            tuning.Nt = Nt;
+            std::size_t mb = std::min<std::size_t>(64, std::max<std::size_t>(1, 1024 / Nt));
+            if (lines) {
+                mb = std::max(line, std::min(2 * line, 512 / Nt));
+            }
+            // few K-columns: smaller tiles until every CU has a work-group or a tile is one wave
+            std::size_t const few = std::max<std::size_t>(1, 64 / Nt);
+            while (!real && mb > few && kcols * ((M + mb - 1) / mb) < 256) {
+                mb = std::max(few, mb / 2);
+            }
+            std::size_t mg = (M + mb - 1) / mb;
+            c.factorization = f;
+            c.Nt = Nt;
+            c.Kb = 1;
+            c.flags = 0;
+            c.lds_pad = nfft >= 32 && (f.size() > 1 || real) ? 16 : 0;
+            for (c.Mb = (M + mg - 1) / mg;
+                 c.Mb > 1 && (c.lds_bytes() > info.local_memory_size / 2 || c.Mb * Nt > 1024);) {
+                ++mg;
+                c.Mb = (M + mg - 1) / mg;
+            }
+            tuning.Mb = c.Mb;
+            if (!real && kcols < 256) {
+                tuning.Kb = 1;
+            }
+            tuning.lds_pad = c.lds_pad;
+            tuning.no_pad = c.lds_pad == 0;
+            tuning.flags = fft1d_per_tile_ids;
+            if (M * Nt * kcols >= 8 * 64 * 256) {
+                tuning.flags |= lines && c.Mb % line == 0
+                                    ? unsigned(fft1d_nontemporal_load | fft1d_nontemporal_store)
+                                    : unsigned(fft1d_xcd_runs);
+            }
+            tuning.has_flags = true;
+        }
+        c.flags = 0;
+    }
 
     if (half_in) {
         if ((all_flags & fft1d_input_f16) && (all_flags & fft1d_input_bf16)) {
@@ -312,7 +608,6 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         throw bad_configuration("lds_pad must be a power of two");
     }
 
-    std::size_t const kcols = c.K_columns(K);
     std::size_t const lds_limit = std::min<std::size_t>(info.local_memory_size, 64 * 1024);
     if (!tuning.Mb) {
         // Shrink the M tile until one K-column tile fits the LDS budget.
@@ -367,15 +662,36 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     c.groups_per_cu = tuning.groups_per_cu;
     if (c.flags & fft1d_prefetch) {
         if (cfg.type == transform_type::c2r || cfg.callbacks || (c.flags & fft1d_mfma) ||
-            direct) {
+            direct || (c.flags & fft1d_per_tile_ids)) {
             throw bad_configuration("Tile prefetching requires a c2c or r2c kernel without "
-                                    "callbacks, MFMA or direct DFT stage");
+                                    "callbacks, MFMA, direct DFT stage or per-tile ids");
+        }
+    }
+    if (c.flags & (fft1d_stage_in | fft1d_stage_out)) {
+        std::size_t const half = cfg.shape[1] / 2 + 1;
+        std::size_t const n_in = cfg.type == transform_type::c2r ? half : N;
+        std::size_t const n_out = cfg.type == transform_type::r2c ? half : N;
+        if ((c.flags & fft1d_stage_in) &&
+            (c.Mb != M || !packed_columns(M, n_in, c.istride) || c.load_function || mfma ||
+             (direct && is_direct_radix(c.factorization[0]) && cfg.type != transform_type::c2r) ||
+             (c.flags & fft1d_prefetch))) {
+            throw bad_configuration("Staged input needs packed columns, one M tile, no load "
+                                    "callback, no MFMA or direct first stage and no tile "
+                                    "prefetching");
+        }
+        if ((c.flags & fft1d_stage_out) &&
+            (c.Mb != M || !packed_columns(M, n_out, c.ostride) || c.store_function)) {
+            throw bad_configuration("Staged output needs packed columns, one M tile and no store "
+                                    "callback");
+        }
+        if (c.lds_bytes() > info.local_memory_size) {
+            throw bad_configuration("Work-group exceeds the local memory size");
         }
     }
     if ((c.flags & fft1d_adjoint) && cfg.type == transform_type::c2c) {
         throw bad_configuration("The adjoint variant applies to real transforms only");
     }
-    c.inplace_unsupported = cfg.type != transform_type::c2c && c.Mb < M;
+    c.inplace_unsupported = cfg.type != transform_type::c2c && (c.Mb < M || inplace_refused);
     return c;
 }
 

@@ -33,6 +33,24 @@
 
 namespace bbfft {
 
+/// Each lane's bytes land at the wave-uniform LDS address plus its lane number times the size
+/// (_NT: non-temporal cache policy, aux bit 1 on gfx950).
+std::string stage_prelude(bool nontemporal) {
+    std::string s = "#ifndef BBFFT_HIP_F4\n#define BBFFT_HIP_F4\n"
+                    "typedef float bbfft_f4 __attribute__((vector_size(16)));\n#endif\n"
+                    "#ifndef BBFFT_WAIT_ALL\n"
+                    "#define BBFFT_WAIT_ALL() __builtin_amdgcn_s_waitcnt(0)\n#endif\n";
+    for (std::string const &n : {std::string("4"), std::string("16")}) {
+        std::string const m = "BBFFT_LDS_DMA" + n + (nontemporal ? "_NT" : "");
+        s += "#ifndef " + m + "\n#define " + m +
+             "(src, dst) __builtin_amdgcn_global_load_lds("
+             "(const __attribute__((address_space(1))) void*)(src), "
+             "(__attribute__((address_space(3))) void*)(dst), " +
+             n + ", 0, " + (nontemporal ? "2" : "0") + ")\n#endif\n";
+    }
+    return s;
+}
+
 namespace {
 
 /// Round to the nearest value with `mant` fraction bits and minimum normal exponent `emin`
@@ -331,7 +349,11 @@ class kernel_gen {
         half_ = real_ && c.N % 2 == 0;
         pairs_ = real_ && c.N % 2 == 1;
         direct_ = c.direct_radix();
-        use_lds_ = L_ > 1 || real_ || direct_;
+        stage_in_ = (c.flags & fft1d_stage_in) != 0;
+        stage_out_ = (c.flags & fft1d_stage_out) != 0;
+        alias_in_ = alias_in_ || stage_in_;
+        alias_out_ = alias_out_ || stage_out_;
+        use_lds_ = L_ > 1 || real_ || direct_ || stage_in_ || stage_out_;
         MG_ = (c.M + c.Mb - 1) / c.Mb;
         if (c.lds_pad) {
             pad_shift_ = 0;
@@ -360,6 +382,9 @@ class kernel_gen {
     std::string generate() {
         if (half_in_) {
             w_.line(half_prelude());
+        }
+        if (stage_in_ || stage_out_) {
+            w_.line(stage_prelude((c_.flags & fft1d_nontemporal_load) != 0));
         }
         emit_tables();
         emit_kernel();
@@ -429,7 +454,7 @@ class kernel_gen {
             std::string const abs = local32_ ? "ibase + (unsigned long)(" + off + ")" : off;
             return std::string(c_.load_function) + "((" + in_type() + "*)in, " + abs + ")";
         }
-        if (c_.flags & fft1d_nontemporal_load) {
+        if (nt_load()) {
             return "ld_nt(tin + " + off + ")";
         }
         return "tin[" + off + "]";
@@ -440,11 +465,15 @@ class kernel_gen {
             std::string const abs = local32_ ? "obase + (unsigned long)(" + off + ")" : off;
             return std::string(c_.store_function) + "(out, " + abs + ", " + val + ");";
         }
-        if (c_.flags & fft1d_nontemporal_store) {
+        if (nt_store()) {
             return "st_nt(tout + " + off + ", " + val + ");";
         }
         return "tout[" + off + "] = " + val + ";";
     }
+
+    /// Streaming hint on the per-element accesses (staged tiles carry it on their copies).
+    bool nt_load() const { return (c_.flags & fft1d_nontemporal_load) && !stage_in_; }
+    bool nt_store() const { return (c_.flags & fft1d_nontemporal_store) && !stage_out_; }
 
     /// Work-group barrier: __syncthreads(), or in fused kernels with lds_barriers a barrier
     /// that orders LDS accesses only (BBFFT_LDS_SYNC, defined by the fused kernel's source).
@@ -600,10 +629,19 @@ class kernel_gen {
                 "* out, unsigned long K) {");
         w_.open("");
         if (use_lds_) {
-            w_.line("__shared__ " + T2() + " lds_buf[" + std::to_string(c_.Mb * c_.Kb * np_) +
-                    "];");
+            std::size_t const eb = 2 * static_cast<std::size_t>(c_.fp);
+            std::size_t const n = std::max({c_.Mb * c_.Kb * np_, (c_.in_tile_bytes() + eb - 1) / eb,
+                                            (c_.out_tile_bytes() + eb - 1) / eb});
+            w_.line("__shared__ " +
+                    std::string(stage_in_ || stage_out_ ? "__attribute__((aligned(16))) " : "") +
+                    T2() + " lds_buf[" + std::to_string(n) + "];");
         }
-        w_.line("const unsigned lid = threadIdx.x;");
+        bool const per_tile_ids = (c_.flags & fft1d_per_tile_ids) != 0;
+        if (per_tile_ids) {
+            w_.line("unsigned lid = threadIdx.x;");
+        } else {
+            w_.line("const unsigned lid = threadIdx.x;");
+        }
         if (direct_) {
             // roots of the direct stage in LDS (read with per-lane indices); the first tile's
             // barrier after the direct stage's input phase orders these writes before any read
@@ -611,9 +649,9 @@ class kernel_gen {
             w_.line("for (unsigned q = lid; q < " + u(direct_) + "; q += " + u(wg) + ") dts[q] = " +
                     dtab_name() + "[q];");
         }
-        w_.line("const unsigned ml = lid % " + u(c_.Mb) + ";");
-        w_.line("const unsigned t = (lid / " + u(c_.Mb) + ") % " + u(c_.Nt) + ";");
-        w_.line("const unsigned kl = lid / " + u(c_.Mb * c_.Nt) + ";");
+        if (!per_tile_ids) {
+            emit_ids();
+        }
         if (pairs_) {
             w_.line("const unsigned long kcols = (K + 1ul) / 2ul;");
         } else {
@@ -621,9 +659,6 @@ class kernel_gen {
         }
         w_.line("const unsigned long ntiles = " + ul(MG_) + " * ((kcols + " + ul(c_.Kb - 1) +
                 ") / " + ul(c_.Kb) + ");");
-        if (use_lds_) {
-            w_.line(T2() + "* col = lds_buf + ml + " + u(c_.Mb * np_) + " * kl;");
-        }
         if (prefetch_) {
             // Stage-0 inputs of the work-group's first tile; each iteration then loads those
             // of the next tile while it transforms the current one.
@@ -638,7 +673,31 @@ class kernel_gen {
             emit_stage0_loads();
             w_.close();
         }
-        w_.open("for (unsigned long tile = blockIdx.x; tile < ntiles; tile += gridDim.x)");
+        std::string first = "blockIdx.x";
+        if (c_.flags & fft1d_xcd_runs) {
+            // block b of a super-block of 8 runs goes to run b % 8 (its XCD); the blocks after
+            // the last whole super-block keep their order
+            std::size_t const run = c_.xcd_run();
+            w_.line("const unsigned xb = blockIdx.x % " + u(8 * run) + ", xs = blockIdx.x - xb;");
+            w_.line("const unsigned first = xs + " + u(8 * run) + " <= gridDim.x ? xs + xb % 8u * " +
+                    u(run) + " + xb / 8u : blockIdx.x;");
+            first = "first";
+        }
+        w_.open("for (unsigned long tile = " + first + "; tile < ntiles; tile += gridDim.x)");
+        if (per_tile_ids) {
+            // The work-item id is opaque in every tile, so the index arithmetic and twiddle
+            // loads that depend on it stay in the tile (the mask restores its range for the
+            // divisions below). Hoisted, they live through the whole tile: 5 x 315 c2r fp64
+            // held 260 registers (one wave per SIMD) instead of 164, 3 x 220 c2r fp32 147
+            // instead of 70.
+            std::size_t range = 1;
+            while (range < wg) {
+                range *= 2;
+            }
+            w_.line("__asm__ volatile(\"\" : \"+v\"(lid));");
+            w_.line("lid &= " + u(range - 1) + ";");
+            emit_ids();
+        }
         emit_tile();
         if (use_lds_) {
             w_.line(sync());
@@ -646,6 +705,16 @@ class kernel_gen {
         w_.close();
         w_.close();
         w_.line("}");
+    }
+
+    /// Coordinates (ml, t, kl) of work-item lid and its LDS column.
+    void emit_ids() {
+        w_.line("const unsigned ml = lid % " + u(c_.Mb) + ";");
+        w_.line("const unsigned t = (lid / " + u(c_.Mb) + ") % " + u(c_.Nt) + ";");
+        w_.line("const unsigned kl = lid / " + u(c_.Mb * c_.Nt) + ";");
+        if (use_lds_) {
+            w_.line(T2() + "* col = lds_buf + ml + " + u(c_.Mb * np_) + " * kl;");
+        }
     }
 
     void emit_body() {
@@ -678,6 +747,9 @@ class kernel_gen {
     /// One (M tile, K tile) of work: `tile` selects it.
     void emit_tile() {
         emit_tile_origin();
+        if (stage_in_) {
+            emit_stage_in();
+        }
         if (c_.type == transform_type::c2r) {
             emit_c2r_pre();
             w_.line(sync());
@@ -701,6 +773,98 @@ class kernel_gen {
         if (c_.type == transform_type::r2c) {
             emit_r2c_post();
         }
+        if (stage_out_) {
+            emit_stage_out();
+        }
+    }
+
+    // Staged tiles (fft1d_stage_in / fft1d_stage_out). The tile's Kb K-columns (pairs: 2 Kb) of
+    // a packed layout are one contiguous run of global memory, whatever M and N are. Its copy in
+    // LDS starts as many words after a 16-byte boundary as the run does, so that both move in
+    // 16-byte pieces except for the words before the run's first boundary and after its last.
+    // The kernels are bound by memory: per-element accesses of short runs (N / radix elements
+    // of M columns) kept too few bytes in flight and, streamed, wrote shared lines more than
+    // once (3 x 220 c2r fp32: 1.6 times the output's bytes). MI355X, about 200 MB in and out,
+    // direct / staged: 3 x 100 c2r fp32 2.4 / 5.0 TB/s, 1 x 512 r2c fp32 4.2 / 5.3, 1 x 100 c2c
+    // fp64 5.3 / 6.0 (the two LDS passes and barriers more cost less than the accesses gain).
+
+    /// `nw`: 32-bit words of the tile's valid columns, `col_bytes` bytes each; `hw`: those before
+    /// the first 16-byte boundary of the run at `g`; `n16`: its whole 16-byte pieces; `sw`: words
+    /// of the LDS copy before it.
+    void emit_stage_words(std::string const &g, std::size_t col_bytes) {
+        std::string const kf = pairs_ ? "2ul * " : "";
+        std::size_t const cols = (pairs_ ? 2 : 1) * c_.Kb;
+        w_.line("const unsigned long kleft = K - " + kf + "k0;");
+        w_.line("const unsigned nw = (kleft < " + ul(cols) + " ? (unsigned)kleft : " + u(cols) +
+                ") * " + u(col_bytes / 4) + ";");
+        w_.line("const unsigned sw = " + stage_shift(g) + ";");
+        w_.line("const unsigned hw = (4u - sw) & 3u;");
+        w_.line("const unsigned n16 = nw < hw ? 0u : (nw - hw) / 4u;");
+    }
+    /// Words between the 16-byte boundary below address `g` and `g`.
+    static std::string stage_shift(std::string const &g) {
+        return "((unsigned)(unsigned long)" + g + " & 15u) / 4u";
+    }
+    /// Moves the words outside the 16-byte pieces, one per work-item.
+    void emit_stage_ends(std::string const &dst, std::string const &src) {
+        w_.line("const unsigned ew = nw - 4u * n16; // at most 3 at either end");
+        std::size_t const wg = c_.work_group_size();
+        std::string const loop = wg >= 6 ? "if (lid < ew)"
+                                         : "for (unsigned q = lid; q < ew; q += " + u(wg) + ")";
+        std::string const q = wg >= 6 ? "lid" : "q";
+        w_.open(loop);
+        w_.line("const unsigned e = " + q + " < hw ? " + q + " : 4u * n16 + " + q + ";");
+        w_.line(dst + "[e] = " + src + "[e];");
+        w_.close();
+    }
+
+    /// Copies the tile's input into LDS with direct global-to-LDS loads: 16 bytes per lane, a
+    /// wave 1 KB of contiguous memory per instruction. Full waves copy.
+    void emit_stage_in() {
+        std::size_t const wg = c_.work_group_size();
+        std::size_t const BL = std::min<std::size_t>(64, wg);     // lanes per copying wave
+        std::size_t const NW = std::max<std::size_t>(1, wg / 64); // copying waves
+        std::size_t const pieces = c_.in_tile_bytes() / 16;
+        std::string const nt = (c_.flags & fft1d_nontemporal_load) ? "_NT" : "";
+        w_.line("// input tile -> LDS");
+        w_.open("");
+        emit_stage_words("gin", c_.istride[2] * in_elem_bytes());
+        w_.line("const float* gs = (const float*)gin;");
+        w_.line("float* ls = (float*)lds_buf + sw;");
+        w_.line("const unsigned ln = lid % 64u, wv = lid / 64u;");
+        std::string const guard = wg % 64 != 0 && wg > 64 ? "wv < " + u(NW) + " && " : "";
+        w_.open("for (unsigned it = 0u; it < " + u((pieces + BL * NW - 1) / (BL * NW)) + "; ++it)");
+        w_.line("const unsigned b = (it * " + u(NW) + " + wv) * " + u(BL) + ";");
+        w_.line("if (" + guard + "b + ln < n16) BBFFT_LDS_DMA16" + nt +
+                "(gs + hw + 4u * (b + ln), ls + hw + 4u * b);");
+        w_.close();
+        emit_stage_ends("ls", "gs");
+        w_.line("BBFFT_WAIT_ALL();");
+        w_.close();
+        w_.line(sync());
+    }
+
+    /// Copies the tile's output from LDS to global memory, 16 bytes per work-item.
+    void emit_stage_out() {
+        std::size_t const wg = c_.work_group_size();
+        std::size_t const pieces = c_.out_tile_bytes() / 16;
+        w_.line("// LDS -> output tile");
+        w_.line(sync());
+        w_.open("");
+        emit_stage_words("gout", c_.ostride[2] * out_elem_bytes());
+        w_.line("float* gs = (float*)gout;");
+        w_.line("const float* ls = (const float*)lds_buf + sw;");
+        w_.open("for (unsigned it = 0u; it < " + u((pieces + wg - 1) / wg) + "; ++it)");
+        w_.line("const unsigned i = it * " + u(wg) + " + lid;");
+        std::string const p = "(bbfft_f4*)(gs + hw + 4u * i)";
+        std::string const v = "*(const bbfft_f4*)(ls + hw + 4u * i)";
+        w_.line("if (i < n16) " +
+                ((c_.flags & fft1d_nontemporal_store)
+                     ? "__builtin_nontemporal_store(" + v + ", " + p + ");"
+                     : "*" + p + " = " + v + ";"));
+        w_.close();
+        emit_stage_ends("gs", "ls");
+        w_.close();
     }
 
     /// Register names q<b>_<i> holding the prefetched stage-0 inputs (butterfly b, input i).
@@ -775,10 +939,20 @@ class kernel_gen {
         if (local32_) {
             // Uniform tile base pointers and 32-bit offsets within the tile: the per-lane
             // address arithmetic stays 32-bit and the base can live in scalar registers.
-            w_.line("const " + in_type() + "* tin = in + m0 + " + kf + "k0 * " +
-                    ul(c_.istride[2]) + ";");
-            w_.line(out_type() + "* tout = out + m0 + " + kf + "k0 * " + ul(c_.ostride[2]) +
-                    ";");
+            // Staged tiles: gin / gout address the tile in global memory, tin / tout its copy
+            // in LDS.
+            w_.line("const " + in_type() + "* " + (stage_in_ ? "gin" : "tin") + " = in + m0 + " +
+                    kf + "k0 * " + ul(c_.istride[2]) + ";");
+            w_.line(out_type() + "* " + (stage_out_ ? "gout" : "tout") + " = out + m0 + " + kf +
+                    "k0 * " + ul(c_.ostride[2]) + ";");
+            if (stage_in_) {
+                w_.line("const " + in_type() + "* tin = (const " + in_type() +
+                        "*)((const float*)lds_buf + " + stage_shift("gin") + ");");
+            }
+            if (stage_out_) {
+                w_.line(out_type() + "* tout = (" + out_type() + "*)((float*)lds_buf + " +
+                        stage_shift("gout") + ");");
+            }
             std::string const kl2 = pairs_ ? "2u * kl" : "kl";
             w_.line("const unsigned ib = ml + " + kl2 + " * " + u(c_.istride[2]) + ";");
             w_.line("const unsigned ob = ml + " + kl2 + " * " + u(c_.ostride[2]) + ";");
@@ -972,9 +1146,7 @@ class kernel_gen {
         } else if (half_) {
             if (vector_real_in()) {
                 std::string p = "((const " + T2() + "*)(tin + ib)) + (" + n + ")";
-                w_.line(v + " = " + ((c_.flags & fft1d_nontemporal_load) ? "ld_nt(" + p + ")"
-                                                                          : "*(" + p + ")") +
-                        ";");
+                w_.line(v + " = " + (nt_load() ? "ld_nt(" + p + ")" : "*(" + p + ")") + ";");
             } else {
                 w_.line(v + " = mk(" + gload(ioff("2u * (" + n + ")")) + ", " +
                         gload(ioff("2u * (" + n + ") + 1u")) + ");");
@@ -992,8 +1164,7 @@ class kernel_gen {
         } else if (half_) {
             if (vector_real_out()) {
                 std::string p = "((" + T2() + "*)(tout + ob)) + (" + n + ")";
-                w_.line((c_.flags & fft1d_nontemporal_store) ? "st_nt(" + p + ", " + y + ");"
-                                                             : "*(" + p + ") = " + y + ";");
+                w_.line(nt_store() ? "st_nt(" + p + ", " + y + ");" : "*(" + p + ") = " + y + ";");
             } else {
                 w_.line(gstore(ooff("2u * (" + n + ")"), y + ".x"));
                 w_.line(gstore(ooff("2u * (" + n + ") + 1u"), y + ".y"));
@@ -1413,7 +1584,7 @@ class kernel_gen {
             if (half_) {
                 w_.line(T2() + " x1 = " + gload(ioff(q)) + ";");
                 w_.line("if (" + q + " == 0u) x1.y = " + f_.lit(0.0) + ";");
-                w_.line(T2() + " x2 = " + gload(ioff(u(H) + " - " + q)) + ";");
+                w_.line(T2() + " x2 = " + gload(ioff(mirrored_pos(b, H))) + ";");
                 if (adjoint()) {
                     // Hermitian fold: halve the non-self-conjugate bins, drop imag(Nyquist)
                     w_.line("if (" + q + " != 0u) { x1 = c_scale(x1, " + f_.lit(0.5) +
@@ -1454,13 +1625,24 @@ class kernel_gen {
             if (half_) {
                 w_.line(lds(q + " % " + u(H)) + " = " + s1 + ";");
                 w_.line("if (" + q + " != 0u && 2u * " + q + " != " + u(H) + ") " +
-                        lds(u(H) + " - " + q) + " = " + s2 + ";");
+                        lds(mirrored_pos(b, H)) + " = " + s2 + ";");
             } else {
                 w_.line(lds(q) + " = " + s1 + ";");
-                w_.line("if (" + q + " != 0u) " + lds(u(c_.N) + " - " + q) + " = " + s2 + ";");
+                w_.line("if (" + q + " != 0u) " + lds(mirrored_pos(b, c_.N)) + " = " + s2 + ";");
             }
             w_.close();
         }
+    }
+
+    /// Index (n - q) mod n of q = t + b Nt, 0 <= q <= n / 2 (only round b = 0 holds q = 0).
+    /// Written as (n - b Nt) - t: for n - (t + b Nt) with a known range of t the LLVM of ROCm
+    /// 7.0 reads LDS address 0.
+    std::string mirrored(std::size_t b, std::size_t n) const {
+        return b ? mirrored_pos(b, n) : "(t == 0u ? 0u : " + mirrored_pos(b, n) + ")";
+    }
+    /// The same without the wrap of q = 0: n - q.
+    std::string mirrored_pos(std::size_t b, std::size_t n) const {
+        return "(" + u(n - b * c_.Nt) + " - t)";
     }
 
     /// r2c: complex FFT output in LDS -> Hermitian half spectrum (reference: sbfft_gen.cpp:180-199
@@ -1491,7 +1673,7 @@ class kernel_gen {
             w_.open("if (active && " + q + " < " + u(Q) + ")");
             if (half_) {
                 w_.line("const " + T2() + " y1 = " + lds(q + " % " + u(H)) + ";");
-                w_.line(T2() + " y2 = " + lds("(" + u(H) + " - " + q + ") % " + u(H)) + ";");
+                w_.line(T2() + " y2 = " + lds(mirrored(b, H)) + ";");
                 w_.line("y2.y = -y2.y;");
                 w_.line("const " + T2() + " a = c_scale(c_add(y2, y1), " + half + ");");
                 w_.line("const " + T2() + " bt = c_mul(c_scale(c_sub(y2, y1), " + half + "), " +
@@ -1515,8 +1697,7 @@ class kernel_gen {
                 }
             } else {
                 w_.line("const " + T2() + " y1 = " + lds(q) + ";");
-                w_.line(T2() + " y2 = " + lds("(" + u(c_.N) + " - " + q + ") % " + u(c_.N)) +
-                        ";");
+                w_.line(T2() + " y2 = " + lds(mirrored(b, c_.N)) + ";");
                 w_.line("y2.y = -y2.y;");
                 // adjoint: doubled non-self-conjugate bins (q >= 1), i.e. no 1/2 there
                 std::string w = adjoint() ? "(" + q + " == 0u ? " + half + " : " +
@@ -1538,7 +1719,7 @@ class kernel_gen {
             w_.open("if (active && " + q + " < " + u(Q) + ")");
             if (half_) {
                 w_.line(gstore(ooff(q), o1));
-                w_.line("if (2u * " + q + " != " + u(H) + ") " + gstore(ooff(u(H) + " - " + q), o2));
+                w_.line("if (2u * " + q + " != " + u(H) + ") " + gstore(ooff(mirrored_pos(b, H)), o2));
             } else {
                 w_.line(gstore(ooff(q), o1));
                 w_.line("if (active_b) " + gstore(ooff(q, 1), o2));
@@ -1570,6 +1751,7 @@ class kernel_gen {
     int direct_ = 0; // radix of the direct DFT stage (0: none)
     bool local32_ = false;
     bool prefetch_ = false;
+    bool stage_in_ = false, stage_out_ = false; // tile copied through LDS (16-byte accesses)
 };
 
 } // namespace

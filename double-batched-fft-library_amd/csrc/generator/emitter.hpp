@@ -12,6 +12,10 @@ namespace bbfft {
 
 /// Complex helper functions shared by all kernels of a source (include-guarded).
 std::string hip_prelude();
+/// Direct global-to-LDS loads (4 and 16 bytes per lane; plain or non-temporal), the wait for
+/// them and the 16-byte vector type of staged tiles (each with its own guard: staged plain and
+/// fused kernels may share a source).
+std::string stage_prelude(bool nontemporal);
 /// One tile of cfg's kernel as `static __device__ void name(in, out, K, tile, lds)` for a
 /// work-group of `group_size` work-items (>= cfg.work_group_size()).
 void generate_fft1d_body(std::ostream &os, fft1d_configuration const &cfg,

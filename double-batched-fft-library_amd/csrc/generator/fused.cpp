@@ -330,32 +330,8 @@ void generate_fused2(std::ostream &os, fused2_configuration const &fc, std::stri
     }
     os << hip_prelude();
     if (fc.stage_words) {
-        // direct global-to-LDS load of one 32-bit word per work-item (the LDS address is the
-        // wave-uniform base plus 4 bytes per lane) and a wait for all outstanding loads
-        os << "#ifndef BBFFT_LDS_DMA4\n"
-              "#define BBFFT_LDS_DMA4(src, dst) __builtin_amdgcn_global_load_lds("
-              "(const __attribute__((address_space(1))) void*)(src), "
-              "(__attribute__((address_space(3))) void*)(dst), 4, 0, 0)\n"
-              "#define BBFFT_WAIT_ALL() __builtin_amdgcn_s_waitcnt(0)\n"
-              "#endif\n";
-        if (fc.stage_load_bytes == 16) {
-            os << "#ifndef BBFFT_LDS_DMA16\n"
-                  "#define BBFFT_LDS_DMA16(src, dst) __builtin_amdgcn_global_load_lds("
-                  "(const __attribute__((address_space(1))) void*)(src), "
-                  "(__attribute__((address_space(3))) void*)(dst), 16, 0, 0)\n"
-                  "#endif\n";
-        }
-        if (fc.stage_load_nt) {
-            // the same loads with the non-temporal cache policy (aux bit 1 on gfx950)
-            os << "#ifndef BBFFT_LDS_DMA4_NT\n"
-                  "#define BBFFT_LDS_DMA4_NT(src, dst) __builtin_amdgcn_global_load_lds("
-                  "(const __attribute__((address_space(1))) void*)(src), "
-                  "(__attribute__((address_space(3))) void*)(dst), 4, 0, 2)\n"
-                  "#define BBFFT_LDS_DMA16_NT(src, dst) __builtin_amdgcn_global_load_lds("
-                  "(const __attribute__((address_space(1))) void*)(src), "
-                  "(__attribute__((address_space(3))) void*)(dst), 16, 0, 2)\n"
-                  "#endif\n";
-        }
+        // direct global-to-LDS loads and the wait for them, shared with staged plain kernels
+        os << stage_prelude(fc.stage_load_nt);
     }
     std::size_t const in_bytes = fc.a.type == transform_type::r2c
                                      ? static_cast<std::size_t>(fc.a.fp)

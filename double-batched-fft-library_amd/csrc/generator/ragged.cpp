@@ -141,8 +141,10 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
             G = std::max(G, t.Mb * t.Nt);
             continue;
         }
+        fft1d_tuning plain;
+        plain.unstaged = true;
         auto b = configure_fft1d(variant_configuration(cfg.fp, M, N, static_cast<direction>(d)),
-                                 info);
+                                 info, plain);
         t.factorization = b.factorization;
         t.Nt = b.Nt;
         int const rmax = *std::max_element(b.factorization.begin(), b.factorization.end());

@@ -155,10 +155,11 @@ bool find_fused_pair(pass_layout const &layout, device_info const &info,
     // 0.1997 ms against 0.2070, c2r 0.2045 against 0.2142 (third pass with plain stores);
     // plain loads were faster where the other pass streams its stores (c2c 32 x 64 x 128 x 128
     // 0.2574 against 0.2654, r2c 256 x 64^3 0.2293 against 0.2307) and in 2-D plans, whose
-    // single kernel then re-reads part of a repeated input from that cache.
+    // single kernel then re-reads part of a repeated input from that cache. Problems small
+    // enough to be launch-bound stay in the caches as a whole: plain loads.
     // BBFFT_FUSE_DMA_NT=on|off overrides.
     char const *nt_env = std::getenv("BBFFT_FUSE_DMA_NT");
-    if (fc.stage_words && !nt_env) {
+    if (fc.stage_words && !nt_env && !small) {
         bool plain_stores = D > 2;
         for (std::size_t i = 0; i < D && plain_stores; ++i) {
             if (i == first || i == first + 1) {

@@ -61,8 +61,14 @@ struct BBFFT_EXPORT fft1d_configuration {
     /// Number of K-columns (or K-column pairs) for a given K.
     std::size_t K_columns(std::size_t K) const;
     std::size_t work_group_size() const { return Mb * Nt * Kb; }
+    /// Bytes of a staged tile's input / output in LDS, with the up to 12 bytes by which it is
+    /// shifted (0 when that side is not staged).
+    std::size_t in_tile_bytes() const;
+    std::size_t out_tile_bytes() const;
     /// Bytes of LDS used by one work-group (stage exchange plus direct-stage root tables).
     std::size_t lds_bytes() const;
+    /// Tiles of one run of fft1d_xcd_runs: whole rows of M tiles.
+    std::size_t xcd_run() const;
     /// Radix of the direct DFT stage (a radix above fft1d_max_register_radix), 0 if none.
     int direct_radix() const;
 };
@@ -94,6 +100,19 @@ enum fft1d_flag : unsigned {
     /// Pays off with a persistent grid (groups_per_cu > 0). c2c and r2c without callbacks;
     /// not with fft1d_mfma.
     fft1d_prefetch = 64u,
+    /// The work-group copies its tile's input (output) through LDS with 16-byte accesses, and
+    /// the stages read (write) the copy. Packed layouts only (Mb = M, K-columns contiguous),
+    /// without a callback on that side; the input side not with MFMA, a direct first stage or
+    /// the load-first tile loop.
+    fft1d_stage_in = 128u,
+    fft1d_stage_out = 256u,
+    /// The work-item's index arithmetic and twiddle loads stay inside the tile loop. A launch
+    /// with one tile per work-group gains nothing from hoisting them out of it, and the hoisted
+    /// values stay in registers through the whole tile.
+    fft1d_per_tile_ids = 512u,
+    /// Work-groups that run on one XCD (every eighth) take consecutive tiles, in runs of a few
+    /// tiles: lines that two neighbouring tiles share meet in that XCD's L2.
+    fft1d_xcd_runs = 1024u,
 };
 
 /// Largest radix a stage computes in registers; a larger (odd) radix runs as a direct DFT stage
@@ -121,6 +140,9 @@ struct BBFFT_EXPORT fft1d_tuning {
     /// Persistent launch: this many work-groups per CU loop over the tiles (0 = one work-group
     /// per tile). Does not change the kernel, only its grid.
     unsigned groups_per_cu = 0;
+    /// Kernels whose tiles cannot be staged by the kernel itself (variants of a ragged kernel):
+    /// no staged tiles, and the tiling of kernels without them.
+    bool unstaged = false;
 };
 
 /// Choose a kernel configuration for a 1-D configuration (dim == 1). `variant` (fft1d_flag

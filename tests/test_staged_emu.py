@@ -1,0 +1,168 @@
+"""Staged tiles, per-tile work-item ids and XCD runs of the plain kernels, on the CPU emulator:
+the same bits as the kernels without them, over packed layouts of odd and even sizes, K
+remainders, tiles of less than 16 bytes and buffers that do not start on 16-byte boundaries."""
+import numpy as np
+import pytest
+
+import bbfft_amd as bb
+import oracle
+from emu import runner
+
+STAGE_IN, STAGE_OUT, PER_TILE_IDS, XCD_RUNS = 128, 256, 512, 1024
+SHAPES = [(1, 64, 37), (3, 60, 11), (5, 35, 7), (1, 16, 9), (7, 9, 5), (2, 512, 3), (1, 27, 130),
+          (1, 3, 2), (1, 2, 1), (17, 33, 3)]
+KINDS = [(0, -1), (0, 1), (1, -1), (2, 1)]  # (type, direction)
+
+
+def _cfg(M, N, K, fp, d, t, inplace=False):
+    cfg = bb.configuration(1, [M, N, K], bb.precision(fp), bb.direction(d),
+                           bb.transform_type(t))
+    cfg.set_strides_default(inplace)
+    return cfg
+
+
+def _tuning(cfg, M, flags):
+    kc = bb.kernel_configuration(cfg)
+    return dict(factorization=kc["factorization"], Nt=kc["Nt"], Mb=M, Kb=min(kc["Kb"], 3),
+                lds_pad=kc["lds_pad"], no_pad=kc["lds_pad"] == 0, flags=flags)
+
+
+def _sizes(M, N, K, t):
+    h = N // 2 + 1
+    return M * (h if t == 2 else N) * K, M * (h if t == 1 else N) * K
+
+
+def _input(N, n, t):
+    x = oracle.uniform_complex(N, n)
+    return x.real.copy() if t == 1 else x
+
+
+@pytest.mark.parametrize("flags", [PER_TILE_IDS, STAGE_IN, STAGE_OUT,
+                                   STAGE_IN | STAGE_OUT | PER_TILE_IDS | XCD_RUNS | 3])
+@pytest.mark.parametrize("t,d", KINDS)
+@pytest.mark.parametrize("fp", [4, 8])
+def test_same_bits_as_direct_access(fp, t, d, flags):
+    for M, N, K in SHAPES:
+        cfg = _cfg(M, N, K, fp, d, t)
+        n_in, n_out = _sizes(M, N, K, t)
+        x = _input(N, n_in, t)
+        plain = runner.run(bb, cfg, x, n_out, tuning=_tuning(cfg, M, 0), grid_cap=2)
+        other = runner.run(bb, cfg, x, n_out, tuning=_tuning(cfg, M, flags), grid_cap=2)
+        assert np.array_equal(plain, other), (M, N, K)
+
+
+@pytest.mark.parametrize("t,d", KINDS)
+@pytest.mark.parametrize("fp", [4, 8])
+def test_buffers_off_the_16_byte_boundary(fp, t, d):
+    """Element-aligned buffers at every offset from a 16-byte boundary: the words before the
+    first and after the last boundary move singly, and nothing outside the tensors changes."""
+    npr, npc = (np.float32, np.complex64) if fp == 4 else (np.float64, np.complex128)
+    real_t, cplx_t = ("float", "float2") if fp == 4 else ("double", "double2")
+    for M, N, K in [(3, 35, 4), (1, 27, 9), (5, 9, 2), (1, 64, 3)]:
+        cfg = _cfg(M, N, K, fp, d, t)
+        tun = _tuning(cfg, M, STAGE_IN | STAGE_OUT | PER_TILE_IDS | 3)
+        kc = bb.kernel_configuration(cfg, tuning=tun)
+        in_t, out_t = (real_t if t == 1 else cplx_t), (real_t if t == 2 else cplx_t)
+        fn = runner.compile_kernel(bb.generate_source(cfg, tuning=tun), kc["name"], in_t, out_t)
+        n_in, n_out = _sizes(M, N, K, t)
+        x = _input(N, n_in, t).astype(npr if t == 1 else npc)
+        ref = runner.run(bb, cfg, x, n_out, tuning=_tuning(cfg, M, 0))
+        kcols = (K + 1) // 2 if t and N % 2 else K
+        grid = -(-kcols // kc["Kb"])
+        # offsets that keep the kernel's element alignment (pairs of reals for even N, M = 1)
+        pair = M == 1 and N % 2 == 0
+        step_in = fp if t == 1 and not pair else 2 * fp
+        step_out = fp if t == 2 and not pair else 2 * fp
+        for oi in range(0, 16, step_in):
+            for oo in range(0, 16, step_out):
+                src = np.zeros(x.nbytes + 32, np.uint8)
+                dst = np.full(ref.nbytes + 48, 0xA5, np.uint8)
+                bi = -src.ctypes.data % 16 + oi
+                bo = -dst.ctypes.data % 16 + oo
+                src[bi:bi + x.nbytes] = x.view(np.uint8).ravel()
+                assert fn(src.ctypes.data + bi, dst.ctypes.data + bo, K, grid,
+                          kc["work_group_size"]) == 0
+                out = dst[bo:bo + ref.nbytes]
+                assert np.array_equal(out, ref.view(np.uint8).ravel()), (M, N, K, oi, oo)
+                assert (dst[:bo] == 0xA5).all() and (dst[bo + ref.nbytes:] == 0xA5).all()
+
+
+@pytest.mark.parametrize("M,N,K,mb", [(17, 20, 5, 9), (40, 16, 3, 16), (9, 64, 40, 4)])
+def test_xcd_runs_cover_every_m_tile(M, N, K, mb):
+    cfg = _cfg(M, N, K, 4, -1, 0)
+    tun = dict(_tuning(cfg, M, PER_TILE_IDS), Mb=mb, Kb=1)
+    x = _input(N, M * N * K, 0)
+    plain = runner.run(bb, cfg, x, M * N * K, tuning=dict(tun, flags=0))
+    for cap in (None, 7):
+        runs = runner.run(bb, cfg, x, M * N * K, tuning=dict(tun, flags=PER_TILE_IDS | XCD_RUNS),
+                          grid_cap=cap)
+        assert np.array_equal(plain, runs)
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+@pytest.mark.parametrize("t,d", [(1, -1), (2, 1)])
+def test_in_place_real_transforms_stage_the_packed_side(fp, t, d):
+    """In place, the real side is padded (not packed): only the spectrum's side is staged."""
+    M, N, K = 3, 20, 40000
+    kc = bb.kernel_configuration(_cfg(M, N, K, fp, d, t, True))
+    flags = int(kc["name"].split("_g")[1].split("_")[0])
+    assert bool(flags & STAGE_OUT) == (t == 1) and bool(flags & STAGE_IN) == (t == 2)
+    K = 5
+    cfg = _cfg(M, N, K, fp, d, t, True)
+    tun = dict(_tuning(cfg, M, flags))
+    H = N // 2 + 1
+    npr, npc = (np.float32, np.complex64) if fp == 4 else (np.float64, np.complex128)
+    buf = np.zeros(M * H * K, npc)
+    rng = np.random.default_rng(3)
+    field = rng.uniform(-1, 1, (K, N, M))
+    spec = np.fft.rfft(field, axis=1)
+    if t == 1:
+        r = buf.view(npr).reshape(K, 2 * H, M)
+        r[:, :N, :] = field
+    else:
+        buf[:] = spec.reshape(-1)
+    runner.run(bb, cfg, None, 0, in_place_buffer=buf, tuning=tun)
+    tol = oracle.tolerance(fp, N)
+    if t == 1:
+        assert oracle.rel_l2(buf, spec.reshape(-1)) <= tol
+    else:
+        assert oracle.rel_l2(buf.view(npr).reshape(K, 2 * H, M)[:, :N, :].ravel() / N,
+                             field.ravel()) <= tol
+
+
+def test_staged_sides_need_packed_columns():
+    def bad(cfg, flags, **kw):
+        with pytest.raises(bb.BadConfiguration):
+            bb.kernel_configuration(cfg, tuning=dict(flags=flags, **kw))
+    cfg = bb.configuration(1, [2, 16, 3], istride=[1, 3, 48], ostride=[1, 3, 48])
+    bad(cfg, STAGE_IN)
+    bad(cfg, STAGE_OUT)
+    cfg = _cfg(4, 16, 3, 4, -1, 0)
+    bad(cfg, STAGE_IN, Mb=2)
+    bad(cfg, STAGE_IN | bb.PREFETCH)
+    bad(cfg, PER_TILE_IDS | bb.PREFETCH)
+    bad(_cfg(1, 67, 3, 4, -1, 0), STAGE_IN)
+    cfg.callbacks = bb.user_module("__device__ float2 ld(float2* p, size_t o) { return p[o]; }",
+                                   "ld")
+    bad(cfg, STAGE_IN)
+    assert "_g" in bb.kernel_configuration(cfg, tuning=dict(flags=STAGE_OUT))["name"]
+
+
+@pytest.mark.skipif(not runner.have_tsan(), reason="no ThreadSanitizer runtime")
+@pytest.mark.parametrize("M,N,K,fp,t,d,inplace", [
+    (3, 60, 7, 4, 0, -1, False), (2, 16, 9, 4, 0, 1, True), (1, 27, 8, 4, 1, -1, False),
+    (3, 20, 5, 4, 1, -1, False), (5, 9, 4, 8, 2, 1, False), (1, 64, 6, 4, 2, 1, False)])
+def test_staged_kernels_are_race_free(M, N, K, fp, t, d, inplace):
+    """Copies in and out share the LDS buffer with the stages' exchange (several tiles per
+    work-group, in place included)."""
+    cfg = _cfg(M, N, K, fp, d, t, inplace)
+    tun = dict(_tuning(cfg, M, STAGE_IN | STAGE_OUT | PER_TILE_IDS | XCD_RUNS), Kb=2)
+    kc = bb.kernel_configuration(cfg, tuning=tun)
+    rt, ct = ("float", "float2") if fp == 4 else ("double", "double2")
+    call = (f'{kc["name"]}((const {rt if t == 1 else ct}*)in, ({rt if t == 2 else ct}*)out, '
+            f'{K}ul)')
+    n_in, n_out = _sizes(M, N, K, t)
+    in_b, out_b = n_in * fp * (1 if t == 1 else 2), n_out * fp * (1 if t == 2 else 2)
+    ok, report = runner.race_check(bb.generate_source(cfg, tuning=tun), call, in_b, out_b, 2,
+                                   kc["work_group_size"], in_place=inplace)
+    assert ok, report[-3000:]
