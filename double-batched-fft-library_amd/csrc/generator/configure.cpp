@@ -58,12 +58,15 @@ std::size_t fft1d_configuration::out_tile_bytes() const {
 }
 
 int fft1d_configuration::direct_radix() const {
-    for (auto f : factorization) {
-        if (is_direct_radix(f)) {
-            return f;
-        }
-    }
-    return 0;
+    int const r = factorization.empty()
+                      ? 0
+                      : *std::max_element(factorization.begin(), factorization.end());
+    return is_direct_radix(r) || (flags & fft1d_direct_matrix) ? r : 0;
+}
+
+std::size_t fft1d_configuration::work_group_size() const {
+    std::size_t const n = Mb * Nt * Kb;
+    return (flags & fft1d_direct_matrix) ? (n + 63) / 64 * 64 : n;
 }
 
 std::size_t fft1d_configuration::xcd_run() const {
@@ -201,6 +204,108 @@ void register_factorizations(std::size_t n, std::vector<int> &cur,
             cur.pop_back();
         }
     }
+}
+
+/**
+ * Tiling of a kernel whose largest radix R (a prime) runs on the matrix cores (emit_direct_matrix):
+ * M tile, K tile and work-items per transform with the least estimated time. Units of work are
+ * 16 columns (m, butterfly, k) by 16 output pairs; the estimate weighs idle columns and units,
+ * M tiles (not staged), resident waves and groups per CU, waves per group and columns per group.
+ * Fitted to 4519 kernels of 24 lengths from 37 x 2 to 509 on MI355X (fp32 and fp64; c2c, r2c and
+ * c2r; about 50 MB in and out): its choice is on average 1.8 % slower than the fastest (at most
+ * 34 %). With it 8 x 509 x 8192 c2c fp32 takes 325 us instead of 960 (vector sums), 8 x 254
+ * fp32 27 instead of 97, 8 x 244 c2r fp64 25 instead of 128 (registers).
+ */
+bool choose_direct_tiling(fft1d_configuration c, std::size_t kcols, device_info const &info,
+                          bool whole_m, fft1d_tuning &out) {
+    std::size_t const n = c.N_fft(), M = c.M;
+    std::size_t const R = static_cast<std::size_t>(
+        *std::max_element(c.factorization.begin(), c.factorization.end()));
+    std::size_t const NR = n / R, h = (R - 1) / 2, KT = (h + 16) / 16;
+    bool const f32 = c.fp == precision::f32;
+    std::size_t const wg_max = std::min<std::size_t>(1024, info.max_work_group_size);
+    // the other stages: as few as possible, radices up to 16
+    if (NR > 1) {
+        std::vector<std::vector<int>> facs;
+        std::vector<int> cur;
+        register_factorizations(NR, cur, facs);
+        if (!facs.empty()) {
+            auto const &f = *std::min_element(facs.begin(), facs.end(), [](auto &a, auto &b) {
+                return a.size() != b.size() ? a.size() < b.size() : a.front() < b.front();
+            });
+            c.factorization.assign(1, static_cast<int>(R));
+            c.factorization.insert(c.factorization.end(), f.begin(), f.end());
+        }
+    }
+    c.lds_pad = 0;
+    c.flags |= fft1d_direct_matrix;
+    bool found = false;
+    double best = 0.0;
+    for (std::size_t mb : {M, std::size_t(16), std::size_t(9), std::size_t(8), std::size_t(4),
+                           std::size_t(3), std::size_t(2)}) {
+        if (mb > M || (mb == M ? M > 32 && !whole_m : whole_m)) {
+            continue;
+        }
+        c.Mb = mb;
+        if (mb < M) { // no staged tiles: their copies need all M columns
+            c.flags &= ~unsigned(fft1d_stage_in | fft1d_stage_out);
+        }
+        for (std::size_t kb : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32}) {
+            for (std::size_t tk : {4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+                c.Kb = kb;
+                c.Nt = NR * tk;
+                std::size_t const wg = c.work_group_size();
+                if ((kb > 1 && kb >= 2 * kcols) || wg > wg_max ||
+                    c.lds_bytes() > info.local_memory_size) {
+                    continue;
+                }
+                std::size_t const cols = mb * kb * NR, CT = (cols + 15) / 16, W = wg / 64;
+                double cost = 0.0, held = 0.0;
+                for (std::size_t k = 1; k <= std::min<std::size_t>(4, KT); ++k) {
+                    std::size_t const rounds = (CT * ((KT + k - 1) / k) + W - 1) / W;
+                    double const t = static_cast<double>(rounds) * (static_cast<double>(k) + 0.35);
+                    if (k == 1 || t < cost) {
+                        cost = t;
+                        held = static_cast<double>(rounds * k);
+                    }
+                }
+                double const regs = 60.0 + held * 16.0 * (f32 && h < 32 ? 1.0 : 2.0);
+                if (regs * static_cast<double>((W + 3) / 4) > 512.0) {
+                    continue;
+                }
+                double const waves = static_cast<double>(W);
+                double const groups = std::floor(info.local_memory_size / double(c.lds_bytes()));
+                double const fit = std::max(
+                    waves, std::floor(4.0 * std::min(8.0, std::floor(512.0 / regs)) / waves) * waves);
+                double const resident = std::min({32.0, waves * groups, fit});
+                double const work = cost * waves * 16.0 / (1.35 * double(cols * KT)) *
+                                    double((M + mb - 1) / mb * mb) / double(M);
+                // share of the matrix instructions whose results are used: below it the sums
+                // stay in vector code (5 x 331 r2c fp64, 0.43: 80 us against 71; 30 x 74 r2c fp32,
+                // 0.30: 22 against 17)
+                double const used = double(cols * (h + 1)) / (256.0 * waves * held);
+                if (used < (R <= 61 ? 0.35 : f32 ? 0.2 : 0.55) && kcols > 64) {
+                    continue;
+                }
+                double const score = 0.414 * std::log(work) * std::min(1.0, double(h) / 40.0) +
+                                     0.177 / resident + (mb < M ? 0.056 : 0.0) -
+                                     0.0788 * std::log2(waves) +
+                                     0.221 * std::min(2.0, 1.0 / groups) +
+                                     0.1024 * std::log2(double(cols) / 16.0);
+                if (!found || score < best) {
+                    found = true;
+                    best = score;
+                    out.factorization = c.factorization;
+                    out.Nt = c.Nt;
+                    out.Mb = mb;
+                    out.Kb = kb;
+                    out.lds_pad = 0;
+                    out.no_pad = true;
+                }
+            }
+        }
+    }
+    return found;
 }
 
 /// Work-items of a launch with whole waves (all M columns in a tile).
@@ -391,37 +496,58 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         // (staged, 1-9 % slower than the estimate's choice)
         bool const keep = !real && cfg.fp == precision::f32 && !half_in && (M == 2 || M == 3) &&
                           r <= 16 && M * Nt <= 512;
-        c.flags = all_flags | (in ? fft1d_stage_in : 0u) | (outp ? fft1d_stage_out : 0u);
         fft1d_tuning const untiled = tuning;
-        bool staged = (in || outp) && (keep || choose_tiling(c, kcols, info, tuning));
-        // Real transforms run in place when one tile holds all M columns: up to 64 columns, 512
-        // work-items and 64 KB of LDS for a single K-column.
+        // Large prime factors on the matrix cores. Radices up to 64 also run in registers, which
+        // stays the faster way for fp32 below 37 (31 x 2 and 31 x 4, 8 columns: equal), for fp64
+        // below 31, and for M tiles up to 61 in fp32 and 41 in fp64 (30 columns: 53 x 2 fp32 36 us
+        // against 44, 37 x 2 fp64 29 against 35; but 53 x 2 fp64 88 against 38).
+        int const large = cfg.fp == precision::f32 ? 37 : 31;
+        bool matrix = static_cast<int>(r) >= large && is_prime(static_cast<unsigned>(r)) &&
+                      std::count(f.begin(), f.end(), static_cast<int>(r)) == 1;
         c.factorization = f;
         c.Nt = Nt;
+        if (!registers) { // the direct stage in vector code, which also fixes in-place use below
+            std::size_t const units = (r - 1) / 2 + 1, per_item = cfg.fp == precision::f32 ? 8 : 6;
+            c.Nt = nfft / r * ((units + per_item - 1) / per_item);
+        }
         c.Mb = M;
         c.Kb = 1;
         c.lds_pad = nfft >= 32 && (f.size() > 1 || real) ? 16 : 0;
         c.flags = 0;
-        bool const whole_m = M <= std::max<std::size_t>(1, std::min<std::size_t>(64, 512 / Nt)) &&
-                             (M == 1 || c.lds_bytes() <= 64 * 1024);
-        inplace_refused = real && registers && !whole_m;
-        if (staged && !keep && !(real && whole_m)) {
+        // Real transforms run in place when one tile holds all M columns: up to 64 columns, 512
+        // work-items and 64 KB of LDS for a single K-column.
+        bool const whole_m =
+            M <= std::max<std::size_t>(1, std::min<std::size_t>(64, 512 / c.Nt)) &&
+            (M == 1 || c.lds_bytes() <= 64 * 1024);
+        inplace_refused = real && !whole_m;
+        c.flags = all_flags | (in ? fft1d_stage_in : 0u) | (outp ? fft1d_stage_out : 0u);
+        matrix = matrix && choose_direct_tiling(c, kcols, info, real && whole_m, tuning) &&
+                 (tuning.Mb == M || r > (cfg.fp == precision::f32 ? 61 : 41));
+        if (!matrix) {
+            tuning = untiled;
+        }
+        bool staged = matrix ? (in || outp) && tuning.Mb == M
+                             : (in || outp) && (keep || choose_tiling(c, kcols, info, tuning));
+        if (staged && !matrix && !keep && !(real && whole_m)) {
             // Tiles above half the LDS leave a CU with nothing to overlap a tile's copies, and
             // tiles of all M columns of few K-columns leave CUs idle: M tiles instead (real
             // transforms that run in place keep all M columns).
             fft1d_configuration t = c;
             t.factorization = tuning.factorization;
-            t.Mb = M;
             t.Kb = tuning.Kb;
             t.lds_pad = tuning.lds_pad;
+            t.flags = 0;
             staged = t.lds_bytes() <= info.local_memory_size / 2 &&
                      (real || M == 1 || kcols >= 256 || M * Nt <= 64);
             if (!staged) {
                 tuning = untiled;
             }
         }
+        if (matrix) {
+            tuning.flags = fft1d_per_tile_ids | fft1d_direct_matrix;
+        }
         if (staged) {
-            tuning.flags = fft1d_per_tile_ids;
+            tuning.flags |= fft1d_per_tile_ids;
             // The copies add two barriers to a work-group's latency: below 8 waves per CU there
             // is too little else to hide it (1 x 315 x 200 fp64, to the spectrum and back: 7.6 us
             // plain, 9.3 staged; x 2000: 14.1 / 15.0; x 6000: 25.7 / 25.1)
@@ -437,11 +563,14 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             c.Mb = M;
             c.Kb = tuning.Kb;
             c.flags = tuning.flags;
-            // shared lines: 32 x 5 x 315 c2r fp32 39.7 us against 43.4, 1 x 512 r2c 49.7 / 50.5
+            // shared lines: 5 x 315 x 15000 c2r fp32 39.7 us against 43.4, 1 x 512 r2c 49.7 / 50.5
             if (tuning.Kb && ((c.in_tile_bytes() && (c.in_tile_bytes() - 12) % 128 != 0) ||
                               (c.out_tile_bytes() && (c.out_tile_bytes() - 12) % 128 != 0))) {
                 tuning.flags |= fft1d_xcd_runs;
             }
+        } else if (matrix) {
+            tuning.flags |= fft1d_xcd_runs;
+            tuning.has_flags = true;
         } else if (registers && !(real && whole_m)) {
             // M tiles. Rows of whole 128-byte lines are streamed, 128 to 256 bytes per tile:
             // 4704 x 80 x 16 fp32 19.3 us (32 columns) against 25.1 before (64 columns, hoisted
@@ -562,6 +691,14 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     if (direct && mfma) {
         throw bad_configuration("The MFMA stage does not combine with a direct DFT stage");
     }
+    if (tuning.has_flags && (tuning.flags & fft1d_direct_matrix)) {
+        int const r = *std::max_element(c.factorization.begin(), c.factorization.end());
+        if (r < 17 || !is_prime(static_cast<unsigned>(r)) ||
+            std::count(c.factorization.begin(), c.factorization.end(), r) != 1) {
+            throw bad_configuration("Matrix sums need one prime radix above 16 as the largest");
+        }
+        direct = r;
+    }
     // The MFMA stage does not use the work-items-per-transform split; later stages set it.
     int const rmax = mfma ? *std::max_element(c.factorization.begin() + 1, c.factorization.end())
                           : *std::max_element(c.factorization.begin(), c.factorization.end());
@@ -618,7 +755,9 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             c.Mb = (M + mg - 1) / mg;
         }
     }
-    if (tuning.Kb) {
+    if (tuning.Kb && (tuning.flags & fft1d_direct_matrix)) {
+        c.Kb = tuning.Kb; // whole waves: K-columns beyond kcols are idle
+    } else if (tuning.Kb) {
         c.Kb = std::min(tuning.Kb, kcols);
     } else {
         std::size_t target = 256;
@@ -673,11 +812,9 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         std::size_t const n_out = cfg.type == transform_type::r2c ? half : N;
         if ((c.flags & fft1d_stage_in) &&
             (c.Mb != M || !packed_columns(M, n_in, c.istride) || c.load_function || mfma ||
-             (direct && is_direct_radix(c.factorization[0]) && cfg.type != transform_type::c2r) ||
              (c.flags & fft1d_prefetch))) {
             throw bad_configuration("Staged input needs packed columns, one M tile, no load "
-                                    "callback, no MFMA or direct first stage and no tile "
-                                    "prefetching");
+                                    "callback, no MFMA and no tile prefetching");
         }
         if ((c.flags & fft1d_stage_out) &&
             (c.Mb != M || !packed_columns(M, n_out, c.ostride) || c.store_function)) {
@@ -686,6 +823,15 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
         if (c.lds_bytes() > info.local_memory_size) {
             throw bad_configuration("Work-group exceeds the local memory size");
+        }
+    }
+    if (c.flags & fft1d_direct_matrix) {
+        std::size_t const span = std::max(c.istride[1], c.ostride[1]) * (N + 2) +
+                                 std::max(c.istride[2], c.ostride[2]) * (2 * c.Kb + 1) + c.Mb;
+        if (span * 2 * static_cast<std::size_t>(cfg.fp) >= (std::size_t(1) << 31) ||
+            c.work_group_size() > wg_max) {
+            throw bad_configuration("Matrix sums need 32-bit tile offsets and a work-group of "
+                                    "whole waves");
         }
     }
     if ((c.flags & fft1d_adjoint) && cfg.type == transform_type::c2c) {

@@ -22,6 +22,7 @@
 #include "roots.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -383,6 +384,11 @@ class kernel_gen {
         if (half_in_) {
             w_.line(half_prelude());
         }
+        if (direct_ && (c_.flags & fft1d_direct_matrix)) {
+            w_.line("#ifndef BBFFT_HIP_D4\n#define BBFFT_HIP_D4\n"
+                    "typedef double bbfft_d4 __attribute__((vector_size(32)));\n#endif");
+            w_.line(stage_prelude(false));
+        }
         if (stage_in_ || stage_out_) {
             w_.line(stage_prelude((c_.flags & fft1d_nontemporal_load) != 0));
         }
@@ -636,8 +642,7 @@ class kernel_gen {
                     std::string(stage_in_ || stage_out_ ? "__attribute__((aligned(16))) " : "") +
                     T2() + " lds_buf[" + std::to_string(n) + "];");
         }
-        bool const per_tile_ids = (c_.flags & fft1d_per_tile_ids) != 0;
-        if (per_tile_ids) {
+        if (per_tile_ids()) {
             w_.line("unsigned lid = threadIdx.x;");
         } else {
             w_.line("const unsigned lid = threadIdx.x;");
@@ -649,7 +654,7 @@ class kernel_gen {
             w_.line("for (unsigned q = lid; q < " + u(direct_) + "; q += " + u(wg) + ") dts[q] = " +
                     dtab_name() + "[q];");
         }
-        if (!per_tile_ids) {
+        if (!per_tile_ids()) {
             emit_ids();
         }
         if (pairs_) {
@@ -684,7 +689,7 @@ class kernel_gen {
             first = "first";
         }
         w_.open("for (unsigned long tile = " + first + "; tile < ntiles; tile += gridDim.x)");
-        if (per_tile_ids) {
+        if (per_tile_ids()) {
             // The work-item id is opaque in every tile, so the index arithmetic and twiddle
             // loads that depend on it stay in the tile (the mask restores its range for the
             // divisions below). Hoisted, they live through the whole tile: 5 x 315 c2r fp64
@@ -712,8 +717,13 @@ class kernel_gen {
         w_.line("const unsigned ml = lid % " + u(c_.Mb) + ";");
         w_.line("const unsigned t = (lid / " + u(c_.Mb) + ") % " + u(c_.Nt) + ";");
         w_.line("const unsigned kl = lid / " + u(c_.Mb * c_.Nt) + ";");
+        if (c_.work_group_size() > c_.Mb * c_.Nt * c_.Kb) {
+            band_ = "inb"; // work-items beyond the tile (whole waves for the matrix cores)
+            w_.line("const bool inb = kl < " + u(c_.Kb) + ";");
+        }
         if (use_lds_) {
-            w_.line(T2() + "* col = lds_buf + ml + " + u(c_.Mb * np_) + " * kl;");
+            w_.line(T2() + "* col = lds_buf + ml + " + u(c_.Mb * np_) + " * " +
+                    (band_.empty() ? "kl;" : "(inb ? kl : 0u);"));
         }
     }
 
@@ -757,7 +767,7 @@ class kernel_gen {
         for (std::size_t s = 0; s < L_; ++s) {
             if (s == 0 && mfma_) {
                 emit_mfma_stage0();
-            } else if (is_direct_radix(c_.factorization[s])) {
+            } else if (direct_ && c_.factorization[s] == direct_) {
                 emit_direct_stage(s);
             } else {
                 emit_stage(s);
@@ -1391,11 +1401,13 @@ class kernel_gen {
         // phase 1
         std::size_t const P1 = NR * U;
         std::size_t const B1 = (P1 + c_.Nt - 1) / c_.Nt;
-        for (std::size_t b = 0; b < B1; ++b) {
-            std::string const x = S + "_" + std::to_string(b);
+        auto open_unit = [&](std::size_t b) {
             w_.open("");
             w_.line("const unsigned du = t + " + u(b * c_.Nt) + ";");
             std::string cond = (b + 1) * c_.Nt > P1 ? "du < " + u(P1) : "";
+            if (!band_.empty()) {
+                cond = cond.empty() ? band_ : band_ + " && " + cond;
+            }
             if (cond.empty()) {
                 w_.open("");
             } else {
@@ -1403,14 +1415,39 @@ class kernel_gen {
             }
             w_.line("const unsigned dj = " + (NR == 1 ? std::string("0u") : "du % " + u(NR)) +
                     ";");
-            w_.line("const unsigned di = " + (NR == 1 ? std::string("du") : "du / " + u(NR)) +
-                    ";");
+            w_.line("unsigned di = " + (NR == 1 ? std::string("du") : "du / " + u(NR)) + ";");
+            if (per_tile_ids()) {
+                w_.line("__asm__ volatile(\"\" : \"+v\"(di)); // as tm of the real passes");
+            }
             // x_{R-i} of unit i = 0 does not exist: its index falls back to x_0's
             w_.line("const unsigned dn1 = dj + di * " + u(NR) + ";");
             w_.line("const unsigned dn2 = di == 0u ? dj : dj + (" + u(R) + " - di) * " + u(NR) +
                     ";");
+        };
+        // a staged tile shares its LDS with the slots: every input is read before any is written
+        bool const reads_first = src_global && alias_in_;
+        if (reads_first) {
+            for (std::size_t b = 0; b < B1; ++b) {
+                std::string const y = std::to_string(b);
+                w_.line(T2() + " dx1_" + y + " = " + f_.zero2() + ", dx2_" + y + " = " +
+                        f_.zero2() + ";");
+                open_unit(b);
+                w_.open("if (active)");
+                emit_global_input("dx1_" + y, "dn1");
+                emit_global_input("dx2_" + y, "dn2");
+                w_.close();
+                w_.close();
+                w_.close();
+            }
+            w_.line(sync());
+        }
+        for (std::size_t b = 0; b < B1; ++b) {
+            open_unit(b);
             w_.line(T2() + " x1 = " + f_.zero2() + ", x2 = " + f_.zero2() + ";");
-            if (src_global) {
+            if (reads_first) {
+                w_.line("x1 = dx1_" + std::to_string(b) + ";");
+                w_.line("x2 = dx2_" + std::to_string(b) + ";");
+            } else if (src_global) {
                 w_.open("if (active)");
                 emit_global_input("x1", "dn1");
                 emit_global_input("x2", "dn2");
@@ -1436,6 +1473,10 @@ class kernel_gen {
             w_.close();
         }
         w_.line(sync());
+        if (c_.flags & fft1d_direct_matrix) {
+            emit_direct_matrix(s, p, dst_global);
+            return;
+        }
         // phase 2
         w_.open("");
         w_.line("const unsigned dj = " + (NR == 1 ? std::string("0u") : "t % " + u(NR)) + ";");
@@ -1553,6 +1594,213 @@ class kernel_gen {
         }
     }
 
+    /**
+     * Phase 2 of a direct stage on the matrix cores: the sums over i are two real matrix
+     * products, C = cos(2 pi i k / R) A and S = sin(2 pi i k / R) B, for the columns
+     * (m, butterfly j, k tile) of the work-group, fp32 by v_mfma_f32_16x16x4_f32 and fp64 by
+     * v_mfma_f64_16x16x4_f64 (accumulation in the kernel's precision). A wave takes 16 columns
+     * (real and imaginary parts as two products) and up to four tiles of 16 output pairs
+     * (k, R - k): per four terms it reads a_i and b_i of its columns and, per tile, the root
+     * (i k) mod R of each lane from the LDS table. x_0 is the term i = 0. The outputs stay in
+     * registers until every wave has read the slots. Long fp32 sums are added up in blocks of 16
+     * terms, so that their rounding error stays below that of two running sums.
+     *
+     * Operand layouts (64 lanes): A row and B column are lane % 16, the inner index is
+     * lane / 16; D element r of a lane is column lane % 16 and row 4 (lane / 16) + r (fp32) or
+     * 4 r + lane / 16 (fp64).
+     */
+    void emit_direct_matrix(std::size_t s, std::size_t p, bool dst_global) {
+        std::size_t const R = c_.factorization[s];
+        std::size_t const NR = nfft_ / R;
+        std::size_t const h = (R - 1) / 2;
+        bool const f32 = c_.fp == precision::f32;
+        std::size_t const KT = (h + 16) / 16;              // tiles of 16 output pairs k = 0..h
+        std::size_t const ncols = c_.Mb * NR * c_.Kb;      // complex columns
+        std::size_t const CT = (ncols + 15) / 16;          // tiles of 16 columns
+        std::size_t const W = c_.work_group_size() / 64;   // waves
+        std::size_t const steps = (h + 4) / 4;             // terms i = 0..h, four at a time
+        // pair tiles per wave and round: few rounds, then many tiles (they share their columns)
+        std::size_t KP = 1, rounds = 0;
+        double best = 0.0;
+        for (std::size_t k = 1; k <= std::min<std::size_t>(4, KT); ++k) {
+            std::size_t const n = (CT * ((KT + k - 1) / k) + W - 1) / W;
+            double const cost = static_cast<double>(n) * (static_cast<double>(k) + 0.35);
+            if (k == 1 || cost < best) {
+                best = cost;
+                KP = k;
+                rounds = n;
+            }
+        }
+        std::size_t const G = (KT + KP - 1) / KP; // waves per column tile
+        bool const blocks = f32 && steps > 8;
+        std::string const vec = f32 ? "bbfft_f4" : "bbfft_d4";
+        std::string const op = f32 ? "__builtin_amdgcn_mfma_f32_16x16x4f32"
+                                   : "__builtin_amdgcn_mfma_f64_16x16x4f64";
+        w_.line("// sums over i on the matrix cores");
+        w_.open("");
+        w_.line("unsigned q4 = lid % 64u / 16u;");
+        w_.line("const unsigned c16 = lid % 16u;");
+        if (per_tile_ids()) {
+            w_.line("__asm__ volatile(\"\" : \"+v\"(q4)); // as tm of the real passes");
+        }
+        auto name = [](char const *v, std::size_t rd) { return v + std::to_string(rd); };
+        auto acc = [](char const *v, std::size_t rd, std::size_t n) {
+            return std::string(v) + std::to_string(rd) + "_" + std::to_string(n);
+        };
+        for (std::size_t rd = 0; rd < rounds; ++rd) {
+            std::string const wu = name("wu", rd), cc = name("cc", rd), cv = name("cv", rd),
+                              cz = name("cz", rd), cj = name("cj", rd), ck = name("ck", rd),
+                              cm = name("cm", rd), cp = name("cp", rd), kg = name("kg", rd);
+            w_.line("const unsigned " + wu + " = lid / 64u + " + u(rd * W) + ";");
+            w_.line("const unsigned " + kg + " = " + wu + " % " + u(G) + " * " + u(16 * KP) + ";");
+            w_.line("const unsigned " + cc + " = " + wu + " / " + u(G) + " * 16u + c16;");
+            // lanes and waves without a column compute the first one and store nothing
+            w_.line("const bool " + cv + " = " + cc + " < " + u(ncols) + ";");
+            w_.line("const unsigned " + cz + " = " + cv + " ? " + cc + " : 0u;");
+            w_.line("const unsigned " + cm + " = " + cz + " % " + u(c_.Mb) + ";");
+            w_.line("const unsigned " + cj + " = " + cz + " / " + u(c_.Mb) + " % " + u(NR) + ";");
+            w_.line("const unsigned " + ck + " = " + cz + " / " + u(c_.Mb * NR) + ";");
+            w_.line(T2() + "* " + cp + " = lds_buf + " + cm + " + " + u(c_.Mb * np_) + " * " + ck +
+                    ";");
+            for (std::size_t n = 0; n < KP; ++n) {
+                for (char const *v : {"Cx", "Cy", "Sx", "Sy"}) {
+                    w_.line(vec + " " + acc(v, rd, n) + " = {0, 0, 0, 0};");
+                    if (blocks) {
+                        w_.line(vec + " t" + acc(v, rd, n) + " = {0, 0, 0, 0};");
+                    }
+                }
+            }
+            w_.open("");
+            for (std::size_t n = 0; n < KP; ++n) {
+                std::string const N = std::to_string(n);
+                w_.line("const unsigned dk" + N + " = " + kg + " + " + u(16 * n) + " + c16;");
+                w_.line("const unsigned ds" + N + " = 4u * dk" + N + " % " + u(R) + ";");
+                w_.line("unsigned dm" + N + " = q4 * dk" + N + " % " + u(R) + ";");
+            }
+            w_.line("unsigned na = " + cj + " + q4 * " + u(NR) + ";");
+            w_.line("unsigned nb = " + cj + " + (" + u(R) + " - q4) * " + u(NR) + ";");
+            auto step = [&](bool first, bool last) {
+                // b_0 does not exist, and neither do terms above h
+                std::string const no_a = last ? "4u * " + u(steps - 1) + " + q4 > " + u(h) : "";
+                std::string const no_b = first ? "q4 == 0u" : no_a;
+                auto term = [&](char const *v, std::string const &n, std::string const &none) {
+                    std::string const idx =
+                        none.empty() ? n : "(" + none + " ? " + cj + " : " + n + ")";
+                    w_.line(T2() + " " + v + " = " + lds_at(cp, idx) + ";");
+                    if (!none.empty()) {
+                        w_.line("if (" + none + ") " + v + " = " + f_.zero2() + ";");
+                    }
+                };
+                term("da", "na", no_a);
+                term("db", "nb", no_b);
+                for (std::size_t n = 0; n < KP; ++n) {
+                    std::string const N = std::to_string(n);
+                    w_.line("const " + T2() + " dw" + N + " = dts[dm" + N + "];");
+                    for (auto [v, root, x] :
+                         {std::array<char const *, 3>{"Cx", ".x", "da.x"}, {"Cy", ".x", "da.y"},
+                          {"Sx", ".y", "db.x"}, {"Sy", ".y", "db.y"}}) {
+                        std::string const a = acc(v, rd, n);
+                        w_.line(a + " = " + op + "(dw" + N + root + ", " + x + ", " + a +
+                                ", 0, 0, 0);");
+                    }
+                    if (!last) {
+                        w_.line("dm" + N + " += ds" + N + ";");
+                        w_.line("dm" + N + " = dm" + N + " >= " + u(R) + " ? dm" + N + " - " +
+                                u(R) + " : dm" + N + ";");
+                    }
+                }
+                if (!last) {
+                    w_.line("na += " + u(4 * NR) + ";");
+                    w_.line("nb -= " + u(4 * NR) + ";");
+                }
+            };
+            w_.open("");
+            step(true, false);
+            w_.close();
+            auto flush = [&](bool last) {
+                for (std::size_t n = 0; n < KP; ++n) {
+                    for (char const *v : {"Cx", "Cy", "Sx", "Sy"}) {
+                        std::string const a = acc(v, rd, n);
+                        w_.line(last ? a + " += t" + a + ";"
+                                     : "t" + a + " += " + a + "; " + a + " = " + vec +
+                                           "{0, 0, 0, 0};");
+                    }
+                }
+            };
+            w_.open("for (unsigned st = 1u; st < " + u(steps - 1) + "; ++st)");
+            step(false, false);
+            if (blocks) {
+                w_.open("if ((st & 3u) == 3u)");
+                flush(false);
+                w_.close();
+            }
+            w_.close();
+            w_.open("");
+            step(false, true);
+            w_.close();
+            if (blocks) {
+                flush(true);
+            }
+            w_.close();
+        }
+        if (!dst_global || alias_out_) {
+            w_.line(sync());
+        }
+        for (std::size_t rd = 0; rd < rounds; ++rd) {
+            std::string const cj = name("cj", rd), ck = name("ck", rd), cm = name("cm", rd);
+            w_.open("if (" + name("cv", rd) + ")");
+            if (dst_global) {
+                // the column's own output offset and activity
+                w_.line("const unsigned ob = " + cm + " + " + (pairs_ ? "2u * " : "") + ck +
+                        " * " + u(c_.ostride[2]) + ";");
+                w_.line("const bool active = k0 + " + ck + " < kcols" +
+                        (MG_ * c_.Mb != c_.M ? " && m0 + " + cm + " < " + ul(c_.M) : "") + ";");
+                if (pairs_) {
+                    w_.line("const bool active_b = active && 2ul * (k0 + " + ck +
+                            ") + 1ul < K;");
+                }
+            }
+            auto store = [&](std::string const &y, std::string const &k) {
+                std::string const n = p == 1 ? cj + " * " + u(R) + " + " + k
+                                             : "(" + cj + " / " + u(p) + ") * " + u(p * R) +
+                                                   " + " + cj + " % " + u(p) + " + (" + k + ") * " +
+                                                   u(p);
+                if (dst_global) {
+                    emit_global_output(y, n);
+                } else {
+                    w_.line(lds_at(name("cp", rd), "(" + n + ")") + " = " + y + ";");
+                }
+            };
+            for (std::size_t n = 0; n < KP; ++n) {
+                for (std::size_t r = 0; r < 4; ++r) {
+                    std::string const e = "[" + std::to_string(r) + "]";
+                    std::string const Cx = acc("Cx", rd, n) + e, Cy = acc("Cy", rd, n) + e,
+                                      Sx = acc("Sx", rd, n) + e, Sy = acc("Sy", rd, n) + e;
+                    w_.open("");
+                    w_.line("const unsigned k = " + name("kg", rd) + " + " +
+                            (f32 ? u(16 * n + r) + " + 4u * q4" : u(16 * n + 4 * r) + " + q4") +
+                            ";");
+                    w_.open("if (k <= " + u(h) + (dst_global ? " && active)" : ")"));
+                    std::string const plus = "mk(" + Cx + " - " + Sy + ", " + Cy + " + " + Sx + ")";
+                    std::string const minus = "mk(" + Cx + " + " + Sy + ", " + Cy + " - " + Sx + ")";
+                    w_.line("const " + T2() + " yk = " + (c_.direction < 0 ? minus : plus) + ";");
+                    w_.line("const " + T2() + " yr = " + (c_.direction < 0 ? plus : minus) + ";");
+                    store("yk", "k");
+                    w_.open("if (k != 0u)");
+                    store("yr", "(" + u(R) + " - k)");
+                    w_.close();
+                    w_.close();
+                    w_.close();
+                }
+            }
+            w_.close();
+        }
+        w_.close();
+        if (!dst_global) {
+            w_.line(sync());
+        }
+    }
+
     /// c2r: Hermitian input -> complex FFT input z in LDS (reference: sbfft_gen.cpp:221-247
     /// for even N, 318-351 for odd N; the imaginary part of the DC bin is ignored).
     void emit_c2r_pre() {
@@ -1560,6 +1808,7 @@ class kernel_gen {
             throw bad_configuration("permuted input rows are not supported for c2r");
         }
         w_.line("// c2r pre-pass");
+        emit_hidden_t();
         std::size_t const H = nfft_;
         std::size_t const Q = half_ ? H / 2 + 1 : (c_.N - 1) / 2 + 1;
         std::size_t const B = (Q + c_.Nt - 1) / c_.Nt;
@@ -1584,7 +1833,7 @@ class kernel_gen {
             if (half_) {
                 w_.line(T2() + " x1 = " + gload(ioff(q)) + ";");
                 w_.line("if (" + q + " == 0u) x1.y = " + f_.lit(0.0) + ";");
-                w_.line(T2() + " x2 = " + gload(ioff(mirrored_pos(b, H))) + ";");
+                w_.line(T2() + " x2 = " + gload(ioff(mirrored_pos(q, b, H))) + ";");
                 if (adjoint()) {
                     // Hermitian fold: halve the non-self-conjugate bins, drop imag(Nyquist)
                     w_.line("if (" + q + " != 0u) { x1 = c_scale(x1, " + f_.lit(0.5) +
@@ -1625,30 +1874,41 @@ class kernel_gen {
             if (half_) {
                 w_.line(lds(q + " % " + u(H)) + " = " + s1 + ";");
                 w_.line("if (" + q + " != 0u && 2u * " + q + " != " + u(H) + ") " +
-                        lds(mirrored_pos(b, H)) + " = " + s2 + ";");
+                        lds(mirrored_pos(q, b, H)) + " = " + s2 + ";");
             } else {
                 w_.line(lds(q) + " = " + s1 + ";");
-                w_.line("if (" + q + " != 0u) " + lds(mirrored_pos(b, c_.N)) + " = " + s2 + ";");
+                w_.line("if (" + q + " != 0u) " + lds(mirrored_pos(q, b, c_.N)) + " = " + s2 + ";");
             }
             w_.close();
         }
     }
 
     /// Index (n - q) mod n of q = t + b Nt, 0 <= q <= n / 2 (only round b = 0 holds q = 0).
-    /// Written as (n - b Nt) - t: for n - (t + b Nt) with a known range of t the LLVM of ROCm
-    /// 7.0 reads LDS address 0.
-    std::string mirrored(std::size_t b, std::size_t n) const {
-        return b ? mirrored_pos(b, n) : "(t == 0u ? 0u : " + mirrored_pos(b, n) + ")";
+    std::string mirrored(std::string const &q, std::size_t b, std::size_t n) const {
+        if (!per_tile_ids()) {
+            return "(" + u(n) + " - " + q + ") % " + u(n);
+        }
+        return b ? mirrored_pos(q, b, n) : "(t == 0u ? 0u : " + mirrored_pos(q, b, n) + ")";
     }
     /// The same without the wrap of q = 0: n - q.
-    std::string mirrored_pos(std::size_t b, std::size_t n) const {
-        return "(" + u(n - b * c_.Nt) + " - t)";
+    std::string mirrored_pos(std::string const &q, std::size_t b, std::size_t n) const {
+        return per_tile_ids() ? "(" + u(n - b * c_.Nt) + " - tm)" : u(n) + " - " + q;
     }
+    /// `tm` = t with its range hidden: where the compiler knows the range of t (per-tile ids
+    /// mask it), the LLVM of ROCm 7.0 turns LDS addresses of the form (constant - t) into 0.
+    void emit_hidden_t() {
+        if (per_tile_ids()) {
+            w_.line("unsigned tm = t;");
+            w_.line("__asm__ volatile(\"\" : \"+v\"(tm));");
+        }
+    }
+    bool per_tile_ids() const { return (c_.flags & fft1d_per_tile_ids) != 0; }
 
     /// r2c: complex FFT output in LDS -> Hermitian half spectrum (reference: sbfft_gen.cpp:180-199
     /// for even N, 275-291 for odd N).
     void emit_r2c_post() {
         w_.line("// r2c post-pass");
+        emit_hidden_t();
         std::size_t const H = nfft_;
         std::size_t const Q = half_ ? H / 2 + 1 : (c_.N - 1) / 2 + 1;
         std::size_t const B = (Q + c_.Nt - 1) / c_.Nt;
@@ -1673,7 +1933,7 @@ class kernel_gen {
             w_.open("if (active && " + q + " < " + u(Q) + ")");
             if (half_) {
                 w_.line("const " + T2() + " y1 = " + lds(q + " % " + u(H)) + ";");
-                w_.line(T2() + " y2 = " + lds(mirrored(b, H)) + ";");
+                w_.line(T2() + " y2 = " + lds(mirrored(q, b, H)) + ";");
                 w_.line("y2.y = -y2.y;");
                 w_.line("const " + T2() + " a = c_scale(c_add(y2, y1), " + half + ");");
                 w_.line("const " + T2() + " bt = c_mul(c_scale(c_sub(y2, y1), " + half + "), " +
@@ -1697,7 +1957,7 @@ class kernel_gen {
                 }
             } else {
                 w_.line("const " + T2() + " y1 = " + lds(q) + ";");
-                w_.line(T2() + " y2 = " + lds(mirrored(b, c_.N)) + ";");
+                w_.line(T2() + " y2 = " + lds(mirrored(q, b, c_.N)) + ";");
                 w_.line("y2.y = -y2.y;");
                 // adjoint: doubled non-self-conjugate bins (q >= 1), i.e. no 1/2 there
                 std::string w = adjoint() ? "(" + q + " == 0u ? " + half + " : " +
@@ -1719,7 +1979,7 @@ class kernel_gen {
             w_.open("if (active && " + q + " < " + u(Q) + ")");
             if (half_) {
                 w_.line(gstore(ooff(q), o1));
-                w_.line("if (2u * " + q + " != " + u(H) + ") " + gstore(ooff(mirrored_pos(b, H)), o2));
+                w_.line("if (2u * " + q + " != " + u(H) + ") " + gstore(ooff(mirrored_pos(q, b, H)), o2));
             } else {
                 w_.line(gstore(ooff(q), o1));
                 w_.line("if (active_b) " + gstore(ooff(q, 1), o2));

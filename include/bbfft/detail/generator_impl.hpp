@@ -60,7 +60,9 @@ struct BBFFT_EXPORT fft1d_configuration {
     bool pairs_k() const;
     /// Number of K-columns (or K-column pairs) for a given K.
     std::size_t K_columns(std::size_t K) const;
-    std::size_t work_group_size() const { return Mb * Nt * Kb; }
+    /// Mb Nt Kb work-items; whole waves of them where the direct stage runs on the matrix cores
+    /// (work-items beyond the tile take part in the barriers, copies and matrix sums only).
+    std::size_t work_group_size() const;
     /// Bytes of a staged tile's input / output in LDS, with the up to 12 bytes by which it is
     /// shifted (0 when that side is not staged).
     std::size_t in_tile_bytes() const;
@@ -69,7 +71,8 @@ struct BBFFT_EXPORT fft1d_configuration {
     std::size_t lds_bytes() const;
     /// Tiles of one run of fft1d_xcd_runs: whole rows of M tiles.
     std::size_t xcd_run() const;
-    /// Radix of the direct DFT stage (a radix above fft1d_max_register_radix), 0 if none.
+    /// Radix of the direct DFT stage (a radix above fft1d_max_register_radix, or with
+    /// fft1d_direct_matrix the largest radix), 0 if none.
     int direct_radix() const;
 };
 
@@ -102,8 +105,8 @@ enum fft1d_flag : unsigned {
     fft1d_prefetch = 64u,
     /// The work-group copies its tile's input (output) through LDS with 16-byte accesses, and
     /// the stages read (write) the copy. Packed layouts only (Mb = M, K-columns contiguous),
-    /// without a callback on that side; the input side not with MFMA, a direct first stage or
-    /// the load-first tile loop.
+    /// without a callback on that side; the input side not with MFMA or the load-first tile
+    /// loop.
     fft1d_stage_in = 128u,
     fft1d_stage_out = 256u,
     /// The work-item's index arithmetic and twiddle loads stay inside the tile loop. A launch
@@ -113,6 +116,9 @@ enum fft1d_flag : unsigned {
     /// Work-groups that run on one XCD (every eighth) take consecutive tiles, in runs of a few
     /// tiles: lines that two neighbouring tiles share meet in that XCD's L2.
     fft1d_xcd_runs = 1024u,
+    /// The sums of the direct stage run on the matrix cores, for the kernel's largest radix if
+    /// that is an odd prime above 16 (once in the factorisation). Work-groups are whole waves.
+    fft1d_direct_matrix = 2048u,
 };
 
 /// Largest radix a stage computes in registers; a larger (odd) radix runs as a direct DFT stage

@@ -226,6 +226,34 @@ template <typename Body> int launch(unsigned grid, unsigned block, Body body) {
 
 } // namespace emu
 
+namespace emu {
+inline double mfma16_a[16][64], mfma16_b[16][64];
+
+/// One v_mfma_{f32,f64}_16x16x4 of a wave: A row / B column = lane % 16, inner index lane / 16;
+/// D item r of lane l = column l % 16, row 4 (l / 16) + r (fp32) or 4 r + l / 16 (fp64). Every
+/// lane of the work-group must call it (two work-group barriers).
+template <typename T, typename V4> V4 mfma_16x16x4(T a, T b, V4 c) {
+    unsigned const lid = cur(), w = lid / 64u, l = lid % 64u;
+    mfma16_a[w][l] = a;
+    mfma16_b[w][l] = b;
+    __syncthreads();
+    V4 d = c;
+    for (unsigned r = 0; r < 4; ++r) {
+        unsigned const i = sizeof(T) == 4 ? 4u * (l / 16u) + r : 4u * r + l / 16u;
+        T s = d[r];
+        for (unsigned k = 0; k < 4; ++k) {
+            s += static_cast<T>(mfma16_a[w][i + 16u * k]) *
+                 static_cast<T>(mfma16_b[w][l % 16u + 16u * k]);
+        }
+        d[r] = s;
+    }
+    __syncthreads();
+    return d;
+}
+} // namespace emu
+#define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu::mfma_16x16x4<float>(a, b, c)
+#define __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, x, y, z) emu::mfma_16x16x4<double>(a, b, c)
+
 #if defined(__clang__)
 namespace emu {
 inline float mfma_a[16][64][8];

@@ -15,6 +15,10 @@ pytestmark = [pytest.mark.gpu,
 SHAPES = [(1, 2), (1, 16), (1, 27), (1, 64), (1, 315), (1, 512), (2, 128), (3, 60), (5, 35),
           (5, 315), (6, 77), (17, 105), (17, 512), (32, 96), (39, 300), (64, 64), (64, 512),
           (70, 20)]
+# lengths whose largest prime factor runs on the matrix cores: one to sixteen tiles of output
+# pairs, more stages, M tiles, idle columns
+MATRIX = [(1, 37), (8, 94), (4, 74), (17, 82), (8, 212), (1, 61), (1, 67), (3, 67), (8, 134),
+          (5, 201), (17, 127), (8, 199), (40, 254), (2, 331), (8, 509), (1, 509)]
 
 
 def _run(M, N, K, fp, t, d, inplace=False, off_in=0, off_out=0):
@@ -77,6 +81,14 @@ def test_untabled_shapes(M, N, t, d, fp):
 
 
 @pytest.mark.parametrize("fp", [4, 8])
+@pytest.mark.parametrize("t,d", [(0, -1), (0, 1), (1, -1), (2, 1)])
+@pytest.mark.parametrize("M,N", MATRIX)
+def test_matrix_sums(M, N, t, d, fp):
+    _run(M, N, (1 << 20) // (M * N) | 1, fp, t, d)
+    _run(M, N, 1, fp, t, d)
+
+
+@pytest.mark.parametrize("fp", [4, 8])
 @pytest.mark.parametrize("t,d", [(0, -1), (1, -1), (2, 1)])
 def test_buffers_off_the_16_byte_boundary(t, d, fp):
     for M, N in [(3, 35), (1, 315), (5, 64)]:
@@ -86,6 +98,6 @@ def test_buffers_off_the_16_byte_boundary(t, d, fp):
 
 @pytest.mark.parametrize("fp", [4, 8])
 @pytest.mark.parametrize("t,d", [(0, -1), (1, -1), (2, 1)])
-@pytest.mark.parametrize("M,N", [(1, 64), (3, 20), (3, 35), (16, 60)])
+@pytest.mark.parametrize("M,N", [(1, 64), (3, 20), (3, 35), (16, 60), (3, 67), (4, 134)])
 def test_in_place(M, N, t, d, fp):
     _run(M, N, (1 << 20) // (M * N) | 1, fp, t, d, inplace=True)

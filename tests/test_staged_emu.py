@@ -141,7 +141,6 @@ def test_staged_sides_need_packed_columns():
     bad(cfg, STAGE_IN, Mb=2)
     bad(cfg, STAGE_IN | bb.PREFETCH)
     bad(cfg, PER_TILE_IDS | bb.PREFETCH)
-    bad(_cfg(1, 67, 3, 4, -1, 0), STAGE_IN)
     cfg.callbacks = bb.user_module("__device__ float2 ld(float2* p, size_t o) { return p[o]; }",
                                    "ld")
     bad(cfg, STAGE_IN)
@@ -166,3 +165,46 @@ def test_staged_kernels_are_race_free(M, N, K, fp, t, d, inplace):
     ok, report = runner.race_check(bb.generate_source(cfg, tuning=tun), call, in_b, out_b, 2,
                                    kc["work_group_size"], in_place=inplace)
     assert ok, report[-3000:]
+
+
+MATRIX = 2048
+MATRIX_CASES = [  # M, N, K, factorisation, work-items per transform, M tile, K tile
+    (1, 67, 5, [67], 64, 1, 2), (2, 134, 3, [67, 2], 32, 2, 1), (2, 134, 3, [2, 67], 32, 2, 1),
+    (4, 212, 3, [53, 4], 16, 4, 1), (3, 67, 9, [67], 64, 3, 2), (2, 37, 7, [37], 32, 2, 2),
+    (4, 127, 3, [127], 16, 4, 2), (5, 17, 3, [17], 32, 2, 1), (2, 469, 3, [7, 67], 224, 2, 1),
+    (2, 509, 2, [509], 32, 2, 1), (3, 67, 7, [67], 8, 3, 3), (5, 74, 3, [37, 2], 12, 5, 2)]
+
+
+@pytest.mark.parametrize("flags", [PER_TILE_IDS, PER_TILE_IDS | STAGE_IN | STAGE_OUT | 3])
+@pytest.mark.parametrize("fp", [4, 8])
+@pytest.mark.parametrize("M,N,K,fac,Nt,Mb,Kb", MATRIX_CASES)
+def test_matrix_sums(M, N, K, fac, Nt, Mb, Kb, fp, flags):
+    """The direct stage on the matrix cores against the FP64 oracle: c2c of the length and the
+    real transforms of twice the length (even) and of the length (odd)."""
+    if flags & STAGE_IN and Mb != M:
+        pytest.skip("staged tiles hold all M columns")
+    tun = dict(factorization=fac, Nt=Nt, Mb=Mb, Kb=Kb, no_pad=True, flags=flags | MATRIX)
+    for t, d, n in [(0, -1, N), (0, 1, N), (1, -1, 2 * N), (2, 1, 2 * N), (1, -1, N), (2, 1, N)]:
+        if n == N and t and N % 2 == 0:
+            continue
+        cfg = _cfg(M, n, K, fp, d, t)
+        n_in, n_out = _sizes(M, n, K, t)
+        x = _input(n, n_in, t)
+        y = runner.run(bb, cfg, x, n_out, tuning=tun, grid_cap=2)
+        ref = oracle.fft(1, cfg.shape, cfg.istride, cfg.ostride, t, d, x)
+        assert oracle.rel_l2(y, ref) <= oracle.tolerance(fp, n), (t, d, n)
+
+
+def test_matrix_sums_are_planned_for_large_primes():
+    for desc, on in [("scfo8.509*8192", True), ("dcfo8.62*1000", True), ("scfo8.62*1000", False),
+                     ("scfo1.74*5000", True), ("scfo8.64*1000", False), ("srfo8.134*900", True)]:
+        kc = bb.kernel_configuration(bb.parse_fft_descriptor(desc + ""))
+        flags = int(kc["name"].split("_g")[1].split("_")[0]) if "_g" in kc["name"] else 0
+        assert bool(flags & MATRIX) == on, desc
+        assert not on or kc["work_group_size"] % 64 == 0
+    cfg = _cfg(2, 64, 3, 4, -1, 0)
+    with pytest.raises(bb.BadConfiguration):
+        bb.kernel_configuration(cfg, tuning=dict(flags=MATRIX))
+    kc = bb.kernel_configuration(_cfg(3, 67, 3, 4, -1, 0), tuning=dict(
+        factorization=[67], Nt=8, Mb=3, Kb=3, no_pad=True, flags=MATRIX))
+    assert kc["work_group_size"] == 128  # 72 work-items, whole waves
