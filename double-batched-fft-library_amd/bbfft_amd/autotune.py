@@ -35,7 +35,9 @@ TABLE_HEADER = ("# Tuned kernel parameters for gfx950 (MI355X), written by "
                 "`python -m bbfft_amd.autotune`.\n"
                 "# precision type N M : factorization Nt Mb Kb lds_pad flags "
                 "[waves_per_eu [groups_per_cu]]"
-                "   # GB/s default -> tuned, descriptor\n")
+                "   # GB/s default -> tuned, descriptor\n"
+                "# Compiled in, an entry with flags 0 and no waves_per_eu is the tiling of a "
+                "staged kernel where the layout is packed.\n")
 
 
 def _divisors(n):

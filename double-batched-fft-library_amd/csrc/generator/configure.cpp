@@ -479,15 +479,83 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     std::size_t const kcols = c.K_columns(K);
 
     bool inplace_refused = false;
+    std::size_t const half = N / 2 + 1;
+    bool const in = packed_columns(M, cfg.type == transform_type::c2r ? half : N, c.istride);
+    bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N, c.ostride);
+    bool const real = cfg.type != transform_type::c2c;
+    std::size_t const eb = 2 * static_cast<std::size_t>(cfg.fp);
+    // Adds the flags of a kernel whose packed sides may be staged; `items`: work-items of the
+    // launch.
+    auto const stage = [&](std::size_t items) {
+        tuning.flags |= fft1d_per_tile_ids;
+        std::size_t const half_eb = half_in ? 4 : eb;
+        std::size_t const bytes =
+            M * K *
+            ((cfg.type == transform_type::r2c ? N * eb / 2
+                                              : (cfg.type == transform_type::c2r ? half : N) * half_eb) +
+             (cfg.type == transform_type::c2r ? N * eb / 2
+                                              : (cfg.type == transform_type::r2c ? half : N) * eb));
+        auto const &f = tuning.factorization;
+        int const r = f.empty() ? 0 : *std::max_element(f.begin(), f.end());
+        if (r <= 32 && bytes <= (real ? 26u : 34u) << 20) {
+            // Data that fits the 32 MB of L2: plain loads find what the last kernel left there,
+            // and streamed stores take the write-back off the kernel's end. The copies' barriers
+            // have nothing to win back, except in real transforms of short rows. To the spectrum
+            // and back in microseconds (copies / plain / plain with streamed stores): 1 x 64 x
+            // 16384 fp32 9.0 / 7.5 / 7.4, 1 x 100 x 5242 fp64 10.8 / 8.9 / 8.1, 8 x 64 x 4096
+            // fp32 12.6 / 12.7 / 10.4; with twice the data 23.3 / 23.1 / 24.0. r2c 8 x 64 x 4096
+            // 10.4 / 9.6 / 8.7, 1 x 64 x 32768 11.9 / 11.7 / 11.0 (10.5: copies, plain loads).
+            if (!c.store_function && (outp || M * eb >= 24)) {
+                tuning.flags |= fft1d_nontemporal_store;
+            }
+            if (real && M * eb < 40 && N < 256) {
+                tuning.flags |= (in && !c.load_function ? fft1d_stage_in : 0u) |
+                                (outp && !c.store_function ? fft1d_stage_out : 0u);
+            }
+            tuning.has_flags = true;
+            return;
+        }
+        // The copies add two barriers to a work-group's latency: below 8 waves per CU there is too
+        // little else to hide it.
+        bool const filled = items >= 8 * 64 * 256;
+        if (in && !c.load_function && filled) {
+            tuning.flags |= fft1d_stage_in | fft1d_nontemporal_load;
+        }
+        if (!c.store_function && (outp || M * eb >= 24) && filled) {
+            tuning.flags |= (outp ? fft1d_stage_out : 0u) | fft1d_nontemporal_store;
+        }
+        tuning.has_flags = true;
+        c.Mb = M;
+        c.Kb = tuning.Kb;
+        c.flags = tuning.flags;
+        // shared lines: 5 x 315 x 15000 c2r fp32 39.7 us against 43.4, 1 x 512 r2c 49.7 / 50.5
+        if (tuning.Kb && ((c.in_tile_bytes() && (c.in_tile_bytes() - 12) % 128 != 0) ||
+                          (c.out_tile_bytes() && (c.out_tile_bytes() - 12) % 128 != 0))) {
+            tuning.flags |= fft1d_xcd_runs;
+        }
+        c.flags = 0;
+    };
+    if (tuning.builtin && tuning.Mb >= M && !mfma && !half_in && tuning.flags == 0 &&
+        !tuning.waves_per_eu) {
+        // A whole-tile entry of the compiled-in table without hints is the tiling of a staged
+        // kernel: 8 x 16 c2c fp32 166 us (524288 K-columns) against 192 (load-first loop), 8 x 512
+        // 176 / 183, 8 x 384 c2r 181 / 233. Its persistent grid, if any, is for launches that give
+        // each work-group 32 tiles or more (8 x 512 fp64: 32768 K-columns 694 us against 711
+        // staged, 8192 182 / 182, 1000 26.4 / 24.6).
+        std::size_t const columns = std::size_t(32) * 256 * tuning.groups_per_cu * tuning.Kb;
+        if ((!in && !outp) || tuning_in.unstaged) {
+            tuning.has_flags = tuning.groups_per_cu != 0; // else the default hints
+        } else if (columns && kcols >= columns) {
+            tuning.flags = fft1d_per_tile_ids;
+        } else {
+            tuning.groups_per_cu = 0;
+            stage(work_items(M, tuning, kcols));
+        }
+    }
     // Shapes without a table entry: when the K-columns of a side are packed, all M columns of a
     // tile sit in LDS and that side moves in 16-byte pieces, streamed past the caches.
     if (!explicit_tuning && tuning.factorization.empty() && info.type == device_type::gpu &&
         !mfma && !tuning_in.unstaged) {
-        std::size_t const half = N / 2 + 1;
-        bool const in = packed_columns(M, cfg.type == transform_type::c2r ? half : N, c.istride);
-        bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N, c.ostride);
-        bool const real = cfg.type != transform_type::c2c;
-        std::size_t const eb = 2 * static_cast<std::size_t>(cfg.fp);
         auto const f = gen::default_factorization(nfft, 16, 16);
         std::size_t const r = static_cast<std::size_t>(*std::max_element(f.begin(), f.end()));
         bool const registers = r <= static_cast<std::size_t>(fft1d_max_register_radix);
@@ -547,34 +615,16 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             tuning.flags = fft1d_per_tile_ids | fft1d_direct_matrix;
         }
         if (staged) {
-            tuning.flags |= fft1d_per_tile_ids;
-            // The copies add two barriers to a work-group's latency: below 8 waves per CU there
-            // is too little else to hide it (1 x 315 x 200 fp64, to the spectrum and back: 7.6 us
-            // plain, 9.3 staged; x 2000: 14.1 / 15.0; x 6000: 25.7 / 25.1)
-            bool const filled = (keep ? M * Nt * kcols : work_items(M, tuning, kcols)) >=
-                                8 * 64 * 256;
-            if (in && !c.load_function && filled) {
-                tuning.flags |= fft1d_stage_in | fft1d_nontemporal_load;
-            }
-            if (!c.store_function && (outp || M * eb >= 24) && filled) {
-                tuning.flags |= (outp ? fft1d_stage_out : 0u) | fft1d_nontemporal_store;
-            }
-            tuning.has_flags = true;
-            c.Mb = M;
-            c.Kb = tuning.Kb;
-            c.flags = tuning.flags;
-            // shared lines: 5 x 315 x 15000 c2r fp32 39.7 us against 43.4, 1 x 512 r2c 49.7 / 50.5
-            if (tuning.Kb && ((c.in_tile_bytes() && (c.in_tile_bytes() - 12) % 128 != 0) ||
-                              (c.out_tile_bytes() && (c.out_tile_bytes() - 12) % 128 != 0))) {
-                tuning.flags |= fft1d_xcd_runs;
-            }
+            stage(keep ? M * Nt * kcols : work_items(M, tuning, kcols));
         } else if (matrix) {
             tuning.flags |= fft1d_xcd_runs;
             tuning.has_flags = true;
         } else if (registers && !(real && whole_m)) {
-            // M tiles. Rows of whole 128-byte lines are streamed, 128 to 256 bytes per tile:
-            // 4704 x 80 x 16 fp32 19.3 us (32 columns) against 25.1 before (64 columns, hoisted
-            // ids), 64 x 512 x 700 63.7 against 99.3. Otherwise neighbouring M tiles share the
+            // M tiles. Rows of whole 128-byte lines are stored past the caches, 128 to 256 bytes
+            // per tile: 4704 x 80 x 16 fp32 20.0 us (32 columns; 25.1 with 64 columns and hoisted
+            // ids, 21.5 with plain stores). Streamed loads as well: 19.4, but data that the last
+            // kernel left in a cache is lost (512 x 64 x 64 to the spectrum and back 13.2 against
+            // 10.5; 8320 x 128 x 32 from HBM 95.6 against 86.6). Otherwise neighbouring M tiles share the
             // lines at their seams: the widest tiles, plain accesses and neighbours on one XCD;
             // 17 x 512 x 2757 fp32 81 us (9 columns) against 323 (6 columns streamed, neighbours
             // on different XCDs) and 130 (9 columns plain, different XCDs).
@@ -611,10 +661,10 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             tuning.lds_pad = c.lds_pad;
             tuning.no_pad = c.lds_pad == 0;
             tuning.flags = fft1d_per_tile_ids;
-            if (M * Nt * kcols >= 8 * 64 * 256) {
-                tuning.flags |= lines && c.Mb % line == 0
-                                    ? unsigned(fft1d_nontemporal_load | fft1d_nontemporal_store)
-                                    : unsigned(fft1d_xcd_runs);
+            if (lines && c.Mb % line == 0) {
+                tuning.flags |= fft1d_nontemporal_store;
+            } else if (M * Nt * kcols >= 8 * 64 * 256) {
+                tuning.flags |= fft1d_xcd_runs;
             }
             tuning.has_flags = true;
         }

@@ -100,6 +100,9 @@ std::map<key_t, fft1d_tuning> const &table() {
             tab = parse(ss.str());
         } else {
             tab = parse(builtin_table);
+            for (auto &e : tab) {
+                e.second.builtin = true;
+            }
         }
     });
     return tab;

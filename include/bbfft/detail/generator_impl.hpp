@@ -146,6 +146,8 @@ struct BBFFT_EXPORT fft1d_tuning {
     /// Persistent launch: this many work-groups per CU loop over the tiles (0 = one work-group
     /// per tile). Does not change the kernel, only its grid.
     unsigned groups_per_cu = 0;
+    /// Entry of the compiled-in table.
+    bool builtin = false;
     /// Kernels whose tiles cannot be staged by the kernel itself (variants of a ragged kernel):
     /// no staged tiles, and the tiling of kernels without them.
     bool unstaged = false;

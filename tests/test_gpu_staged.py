@@ -101,3 +101,13 @@ def test_buffers_off_the_16_byte_boundary(t, d, fp):
 @pytest.mark.parametrize("M,N", [(1, 64), (3, 20), (3, 35), (16, 60), (3, 67), (4, 134)])
 def test_in_place(M, N, t, d, fp):
     _run(M, N, (1 << 20) // (M * N) | 1, fp, t, d, inplace=True)
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+@pytest.mark.parametrize("t,d", [(0, -1), (1, -1), (2, 1)])
+@pytest.mark.parametrize("M,N", [(8, 16), (8, 32), (8, 60), (8, 64), (8, 105), (8, 243), (8, 256),
+                                 (8, 384), (8, 512), (1, 64), (1, 128), (4, 512)])
+def test_data_in_and_beyond_the_l2(M, N, t, d, fp):
+    """Tiles of the tuning table and of the estimate, direct (data that fits the L2) and staged."""
+    for elems in (1 << 14, 1 << 20, 5 << 20):
+        _run(M, N, elems // (M * N) | 1, fp, t, d)

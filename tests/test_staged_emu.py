@@ -208,3 +208,25 @@ def test_matrix_sums_are_planned_for_large_primes():
     kc = bb.kernel_configuration(_cfg(3, 67, 3, 4, -1, 0), tuning=dict(
         factorization=[67], Nt=8, Mb=3, Kb=3, no_pad=True, flags=MATRIX))
     assert kc["work_group_size"] == 128  # 72 work-items, whole waves
+
+
+def test_tiles_are_staged_beyond_the_l2():
+    """Data up to 34 MB (real transforms 26 MB) is accessed directly with streamed stores; real
+    transforms of short rows and larger data are staged; layouts that are not packed are not."""
+    def flags(desc, strides=None):
+        cfg = bb.parse_fft_descriptor(desc)
+        if strides:
+            cfg.istride, cfg.ostride = strides
+        kc = bb.kernel_configuration(cfg)
+        return int(kc["name"].split("_g")[1].split("_")[0]) if "_g" in kc["name"] else 0
+    staged = STAGE_IN | STAGE_OUT
+    for desc, want in [("scfo8.256*1000", 0), ("scfo8.256*1100", staged), ("dcfo3.100*3500", 0),
+                       ("dcfo3.100*3800", staged), ("srfo8.64*6000", 0),
+                       ("srfo8.64*6800", staged), ("srfo1.64*1000", staged),
+                       ("srfo1.512*1000", 0), ("dcfo8.512*500", staged),
+                       ("dcfo8.512*8192", 0)]:
+        f = flags(desc)
+        assert f & staged == want and f & PER_TILE_IDS, desc
+    assert flags("scfo8.256*1000") & 3 == 2 and flags("scfo8.256*1100") & 3 == 3
+    padded = [1, 9, 9 * 256]
+    assert flags("scfo8.256*1100", (padded, padded)) & staged == 0
