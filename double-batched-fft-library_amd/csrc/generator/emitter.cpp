@@ -818,7 +818,7 @@ class kernel_gen {
     /// Moves the words outside the 16-byte pieces, one per work-item.
     void emit_stage_ends(std::string const &dst, std::string const &src) {
         w_.line("const unsigned ew = nw - 4u * n16; // at most 3 at either end");
-        std::size_t const wg = c_.work_group_size();
+        std::size_t const wg = std::max(group_size_, c_.work_group_size());
         std::string const loop = wg >= 6 ? "if (lid < ew)"
                                          : "for (unsigned q = lid; q < ew; q += " + u(wg) + ")";
         std::string const q = wg >= 6 ? "lid" : "q";
@@ -831,7 +831,7 @@ class kernel_gen {
     /// Copies the tile's input into LDS with direct global-to-LDS loads: 16 bytes per lane, a
     /// wave 1 KB of contiguous memory per instruction. Full waves copy.
     void emit_stage_in() {
-        std::size_t const wg = c_.work_group_size();
+        std::size_t const wg = std::max(group_size_, c_.work_group_size());
         std::size_t const BL = std::min<std::size_t>(64, wg);     // lanes per copying wave
         std::size_t const NW = std::max<std::size_t>(1, wg / 64); // copying waves
         std::size_t const pieces = c_.in_tile_bytes() / 16;
@@ -856,7 +856,7 @@ class kernel_gen {
 
     /// Copies the tile's output from LDS to global memory, 16 bytes per work-item.
     void emit_stage_out() {
-        std::size_t const wg = c_.work_group_size();
+        std::size_t const wg = std::max(group_size_, c_.work_group_size());
         std::size_t const pieces = c_.out_tile_bytes() / 16;
         w_.line("// LDS -> output tile");
         w_.line(sync());

@@ -26,9 +26,9 @@ namespace {
 
 /// Work-items per work-group of the persistent kernel (at least this many).
 constexpr std::size_t ragged_min_group = 256;
-/// LDS budget of one variant: 160 KB / 5, so that the five work-groups per CU that the
-/// occupancy target (5 waves per SIMD, 4 waves per group) allows also fit in LDS.
-constexpr std::size_t ragged_lds_limit = 32 * 1024;
+/// LDS budget of one variant: 160 KB / 6, so that the six work-groups per CU that the occupancy
+/// target (6 waves per SIMD, 4 waves per group) allows also fit in LDS.
+constexpr std::size_t ragged_lds_limit = 26 * 1024;
 /// Largest radix of a variant. All variants share one kernel, whose register allocation is the
 /// largest of the variants', so one wide radix would lower the occupancy of every job.
 constexpr int ragged_radix_max = 12;
@@ -167,6 +167,15 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
         auto const &[N, M, d] = keys[v];
         fft1d_tuning &t = tune[v];
         t.Kb = std::max<std::size_t>(1, G / (t.Mb * t.Nt));
+        if (t.Mb >= M) {
+            // The tiles of a job are packed: staged through LDS. 256 jobs of the serving mix (7.4
+            // GB in and out) 1.50 ms against 1.70 with per-element accesses; copying the next
+            // tile's input ahead into a second buffer halves the work-groups per CU: 1.67.
+            // Streamed loads gain 1 % there and lose what a cache holds of smaller batches (64
+            // jobs of 512 and 500 points, 0.35 GB: 82 us plain, 94 streamed, 93 per element).
+            t.flags |= fft1d_stage_in | fft1d_stage_out;
+            t.flags &= ~unsigned(fft1d_nontemporal_load);
+        }
         fft1d_configuration c;
         for (;;) {
             c = configure_fft1d(variant_configuration(cfg.fp, M, N, static_cast<direction>(d)),
@@ -189,7 +198,7 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
     }
     rk.group_size = G;
     // occupancy target (BBFFT_RAGGED_WAVES overrides it for measurements)
-    rk.waves_per_eu = cfg.fp == precision::f32 ? 5u : 0u;
+    rk.waves_per_eu = cfg.fp == precision::f32 ? 6u : 0u;
     if (char const *w = std::getenv("BBFFT_RAGGED_WAVES")) {
         rk.waves_per_eu = static_cast<unsigned>(std::atoi(w));
     }
@@ -261,10 +270,12 @@ std::vector<std::uint64_t> ragged_job_table(ragged_configuration const &cfg,
         first[g] = t;
     }
     // job holding each first tile: the last position whose first tile is <= it
+    std::size_t q = 0;
     for (std::size_t g = 0; g < grid; ++g) {
-        auto it = std::upper_bound(rk.tile_begin.begin(), rk.tile_begin.end() - 1, first[g]);
-        pos[g] = static_cast<std::uint64_t>(std::max<std::ptrdiff_t>(
-            0, (it - rk.tile_begin.begin()) - 1));
+        while (q + 1 < n && rk.tile_begin[q + 1] <= first[g]) {
+            ++q;
+        }
+        pos[g] = q;
     }
     return table;
 }
@@ -277,14 +288,18 @@ void generate_ragged(std::ostream &os, ragged_kernel_configuration const &rk,
     std::string const n = name.empty() ? rk.identifier() : std::string(name);
     std::string const T2 = rk.fp == precision::f32 ? "float2" : "double2";
     os << hip_prelude();
+    if (std::any_of(rk.variants.begin(), rk.variants.end(),
+                    [](auto const &c) { return (c.flags & fft1d_stage_in) != 0; })) {
+        os << stage_prelude(false);
+    }
     for (std::size_t v = 0; v < rk.variants.size(); ++v) {
         generate_fft1d_body(os, rk.variants[v], variant_name(n, v), rk.group_size);
     }
     std::size_t const lds_elems = std::max<std::size_t>(1, rk.lds_bytes() / (2 * static_cast<std::size_t>(rk.fp)));
     // One kernel holds every variant, so its register allocation follows the heaviest one;
-    // for fp32 variants (radix <= 12) the allocator reaches 5 waves per SIMD (96 VGPRs)
-    // without spilling when asked to (measured on MI355X for the 4096-job serving mix: 78.4 ms
-    // against 85.4 ms with radix <= 16 at 4 waves).
+    // for fp32 variants (radix <= 12) the allocator reaches 6 waves per SIMD (80 VGPRs) when
+    // asked to (256 jobs of the serving mix, staged: 1.49 ms against 1.51 at 5 waves; 7 and 8
+    // waves 1.49).
     std::string const occupancy =
         rk.waves_per_eu ? " __attribute__((amdgpu_waves_per_eu(" +
                               std::to_string(rk.waves_per_eu) + ")))"
@@ -293,7 +308,7 @@ void generate_ragged(std::ostream &os, ragged_kernel_configuration const &rk,
        << occupancy << " " << n
        << "(const " << T2 << "* in, " << T2
        << "* out, const unsigned long* table, unsigned long njobs) {\n"
-       << "  __shared__ " << T2 << " lds_buf[" << lds_elems << "];\n"
+       << "  __shared__ __attribute__((aligned(16))) " << T2 << " lds_buf[" << lds_elems << "];\n"
        << "  const unsigned long* first = table + 5ul * njobs + 1ul;\n"
        << "  const unsigned long* pos = first + gridDim.x + 1ul;\n"
        << "  const unsigned long tend = first[blockIdx.x + 1u];\n"

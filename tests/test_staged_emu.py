@@ -230,3 +230,24 @@ def test_tiles_are_staged_beyond_the_l2():
     assert flags("scfo8.256*1000") & 3 == 2 and flags("scfo8.256*1100") & 3 == 3
     padded = [1, 9, 9 * 256]
     assert flags("scfo8.256*1100", (padded, padded)) & staged == 0
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+def test_ragged_variants_stage_whole_tiles(fp):
+    """A ragged kernel of staged variants (all M columns in a tile) and an M-tiled one, jobs at
+    odd offsets."""
+    from bbfft_amd import ragged
+    jobs, off = [], 1
+    for M, N, K, d in [(3, 20, 5, -1), (200, 12, 2, 1), (1, 27, 9, -1), (2, 16, 1, 1), (1, 5, 3, -1)]:
+        jobs.append(ragged.Job(M, N, K, d, off, off + 2))
+        off += M * N * K + 1
+    tiles = [ragged.variant_configuration(jobs, v, fp)["Mb"] for v in ragged.job_variants(jobs, fp)]
+    assert tiles[0] == 3 and tiles[1] < 200
+    x = oracle.uniform_complex(9, off + 4)
+    y = runner.run_ragged(ragged, jobs, x, off + 4, precision=fp, grid=3)
+    for j in jobs:
+        st = [1, j.M, j.M * j.N]
+        ref = oracle.fft(1, [j.M, j.N, j.K], st, st, 0, j.direction,
+                         x[j.in_offset:j.in_offset + j.elements])
+        assert oracle.rel_l2(y[j.out_offset:j.out_offset + j.elements],
+                             ref) <= oracle.tolerance(fp, j.N), j
