@@ -844,6 +844,25 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         default_hints = fft1d_nontemporal_load | fft1d_nontemporal_store;
     }
     c.flags = (tuning.has_flags ? tuning.flags : default_hints) | variant;
+    if (half_in && !explicit_tuning && info.type == device_type::gpu && c.Mb == M) {
+        // Half-precision input: four bytes per element leave the loads cheap and their lines
+        // shared by neighbouring accesses, so they go through the caches, element by element; the
+        // output is staged beyond the 32 MB of L2 (on the matrix cores, whose tiles take more of a
+        // CU, beyond 1 GB: 4 x 512 x 262144 1050 us against 1097 direct, x 16384 68 / 65, 16 x 384
+        // x 3000 62 / 46). MI355X, vector kernels, streamed loads before: 4 x 512 x 262144 f16
+        // 1086 -> 1026 us, 8 x 64 x 60000 62 -> 54, 16 x 384 x 3000 65 -> 43.
+        c.flags = variant | fft1d_per_tile_ids;
+        if (outp || M * eb >= 24) {
+            c.flags |= fft1d_nontemporal_store;
+        }
+        if (outp && M * N * K * (4 + eb) > (mfma ? std::size_t(1) << 30 : std::size_t(34) << 20)) {
+            unsigned const plain = c.flags;
+            c.flags |= fft1d_stage_out | fft1d_xcd_runs;
+            if (c.lds_bytes() > info.local_memory_size) {
+                c.flags = plain;
+            }
+        }
+    }
     if (tuning.waves_per_eu > 8) {
         throw bad_configuration("waves_per_eu must be 0..8");
     }

@@ -251,3 +251,12 @@ def test_ragged_variants_stage_whole_tiles(fp):
                          x[j.in_offset:j.in_offset + j.elements])
         assert oracle.rel_l2(y[j.out_offset:j.out_offset + j.elements],
                              ref) <= oracle.tolerance(fp, j.N), j
+
+
+@pytest.mark.parametrize("mfma", [False, True])
+def test_half_input_stages_its_output_only(mfma):
+    for K, staged in [(1000, False), (40000, not mfma), (100000, True)]:
+        kc = bb.half_input_kernel_configuration(f"scfo4.512*{K}", "f16", mfma)
+        flags = int(kc["name"].split("_g")[1].split("_")[0])
+        assert bool(flags & STAGE_OUT) == staged and not flags & STAGE_IN
+        assert flags & PER_TILE_IDS and flags & 3 == 2
