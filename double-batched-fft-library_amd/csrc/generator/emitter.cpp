@@ -1783,7 +1783,12 @@ class kernel_gen {
                     w_.open("if (k <= " + u(h) + (dst_global ? " && active)" : ")"));
                     std::string const plus = "mk(" + Cx + " - " + Sy + ", " + Cy + " + " + Sx + ")";
                     std::string const minus = "mk(" + Cx + " + " + Sy + ", " + Cy + " - " + Sx + ")";
-                    w_.line("const " + T2() + " yk = " + (c_.direction < 0 ? minus : plus) + ";");
+                    // output 0 has no sine sum: its zero roots turn infinite inputs into NaN
+                    std::string const yk = c_.direction < 0 ? minus : plus;
+                    w_.line("const " + T2() + " yk = " +
+                            (n == 0 && r == 0 ? "k == 0u ? mk(" + Cx + ", " + Cy + ") : " + yk
+                                              : yk) +
+                            ";");
                     w_.line("const " + T2() + " yr = " + (c_.direction < 0 ? plus : minus) + ";");
                     store("yk", "k");
                     w_.open("if (k != 0u)");
