@@ -69,6 +69,17 @@ std::size_t fft1d_configuration::work_group_size() const {
     return (flags & fft1d_direct_matrix) ? (n + 63) / 64 * 64 : n;
 }
 
+bool fft1d_configuration::local_offsets() const {
+    std::size_t const kspan = (pairs_k() ? 2 : 1) * Kb + 1;
+    std::size_t const eb = 2 * static_cast<std::size_t>(fp); // largest element size
+    for (auto const &s : {istride, ostride}) {
+        if ((Mb + (N + 2) * s[1] + kspan * s[2]) * eb >= (std::size_t(1) << 31)) {
+            return false;
+        }
+    }
+    return true;
+}
+
 std::size_t fft1d_configuration::xcd_run() const {
     std::size_t const mg = (M + Mb - 1) / Mb;
     return mg * std::max<std::size_t>(1, 16 / mg);
@@ -214,7 +225,8 @@ void register_factorizations(std::size_t n, std::vector<int> &cur,
  * Fitted to 4519 kernels of 24 lengths from 37 x 2 to 509 on MI355X (fp32 and fp64; c2c, r2c and
  * c2r; about 50 MB in and out): its choice is on average 1.8 % slower than the fastest (at most
  * 34 %). With it 8 x 509 x 8192 c2c fp32 takes 325 us instead of 960 (vector sums), 8 x 254
- * fp32 27 instead of 97, 8 x 244 c2r fp64 25 instead of 128 (registers).
+ * fp32 27 instead of 97, 8 x 244 c2r fp64 25 instead of 128 (registers). None is found where a
+ * tile's extent needs 64-bit offsets.
  */
 bool choose_direct_tiling(fft1d_configuration c, std::size_t kcols, device_info const &info,
                           bool whole_m, fft1d_tuning &out) {
@@ -255,7 +267,7 @@ bool choose_direct_tiling(fft1d_configuration c, std::size_t kcols, device_info 
                 c.Kb = kb;
                 c.Nt = NR * tk;
                 std::size_t const wg = c.work_group_size();
-                if ((kb > 1 && kb >= 2 * kcols) || wg > wg_max ||
+                if ((kb > 1 && kb >= 2 * kcols) || wg > wg_max || !c.local_offsets() ||
                     c.lds_bytes() > info.local_memory_size) {
                     continue;
                 }
@@ -895,10 +907,7 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
     }
     if (c.flags & fft1d_direct_matrix) {
-        std::size_t const span = std::max(c.istride[1], c.ostride[1]) * (N + 2) +
-                                 std::max(c.istride[2], c.ostride[2]) * (2 * c.Kb + 1) + c.Mb;
-        if (span * 2 * static_cast<std::size_t>(cfg.fp) >= (std::size_t(1) << 31) ||
-            c.work_group_size() > wg_max) {
+        if (!c.local_offsets() || c.work_group_size() > wg_max) {
             throw bad_configuration("Matrix sums need 32-bit tile offsets and a work-group of "
                                     "whole waves");
         }

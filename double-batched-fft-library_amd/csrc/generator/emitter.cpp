@@ -363,16 +363,10 @@ class kernel_gen {
             }
         }
         np_ = (c.lds_pad ? (nfft_ - 1) + (nfft_ - 1) / c.lds_pad : nfft_ - 1) + 1;
-        // 32-bit offsets within a tile when the tile's extent fits comfortably; callbacks,
-        // which take absolute offsets, get the tile's uniform 64-bit base plus the 32-bit
-        // offset within the tile
-        std::size_t const kspan = (pairs_ ? 2 : 1) * c.Kb + 1;
-        std::size_t const nspan = c.N + 2;
-        std::size_t const ext_in = c.Mb + nspan * c.istride[1] + kspan * c.istride[2];
-        std::size_t const ext_out = c.Mb + nspan * c.ostride[1] + kspan * c.ostride[2];
-        std::size_t const eb = 2 * static_cast<std::size_t>(c.fp); // largest element size
-        local32_ =
-            ext_in * eb < (std::size_t(1) << 31) && ext_out * eb < (std::size_t(1) << 31);
+        // 32-bit offsets within a tile when the tile's extent fits; callbacks, which take
+        // absolute offsets, get the tile's uniform 64-bit base plus the 32-bit offset within the
+        // tile
+        local32_ = c.local_offsets();
         half_in_ = (c.flags & (fft1d_input_f16 | fft1d_input_bf16)) != 0;
         bf16_ = (c.flags & fft1d_input_bf16) != 0;
         mfma_ = (c.flags & fft1d_mfma) != 0;

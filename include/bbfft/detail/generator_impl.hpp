@@ -69,6 +69,9 @@ struct BBFFT_EXPORT fft1d_configuration {
     std::size_t out_tile_bytes() const;
     /// Bytes of LDS used by one work-group (stage exchange plus direct-stage root tables).
     std::size_t lds_bytes() const;
+    /// Whether offsets within a tile fit 32 bits (byte offsets below 2^31 on both sides): the
+    /// kernel then adds them to a uniform 64-bit tile address, otherwise every offset has 64 bits.
+    bool local_offsets() const;
     /// Tiles of one run of fft1d_xcd_runs: whole rows of M tiles.
     std::size_t xcd_run() const;
     /// Radix of the direct DFT stage (a radix above fft1d_max_register_radix, or with
@@ -117,7 +120,8 @@ enum fft1d_flag : unsigned {
     /// tiles: lines that two neighbouring tiles share meet in that XCD's L2.
     fft1d_xcd_runs = 1024u,
     /// The sums of the direct stage run on the matrix cores, for the kernel's largest radix if
-    /// that is an odd prime above 16 (once in the factorisation). Work-groups are whole waves.
+    /// that is an odd prime above 16 (once in the factorisation). Work-groups are whole waves, and
+    /// offsets within a tile have 32 bits.
     fft1d_direct_matrix = 2048u,
 };
 

@@ -39,3 +39,55 @@ def test_matrix_sums_of_values_that_are_not_finite(M, N, fac, Nt, Kb, fp, bad):
             for part in (np.real, np.imag):
                 assert np.array_equal(np.isnan(part(y[0])), np.isnan(part(y[1]))), (d, at)
                 assert np.array_equal(np.isinf(part(y[0])), np.isinf(part(y[1]))), (d, at)
+
+
+def _flags(kc):
+    return int(kc["name"].split("_g")[1].split("_")[0]) if "_g" in kc["name"] else 0
+
+
+@pytest.mark.parametrize("desc,p", [
+    ("scfo1.509x509x509", 2), ("dcfo1.331x331x331", 2), ("scfo1024x1024x67", 2),
+    ("dcfo512x512x131", 2), ("scfo640x640x166", 2), ("dcfo2048x2048x47", 2),
+    ("scfo1048576.67", 0), ("srfo3.243x315x131*6", 2)])
+def test_large_prime_factors_far_apart_are_planned(desc, p):
+    """Rows so far apart that a tile may need 64-bit offsets: the sums of a large prime then stay
+    in vector code or registers, which have such offsets, instead of on the matrix cores."""
+    cfg = bb.parse_fft_descriptor(desc)
+    kc = bb.kernel_configuration(cfg, p)
+    rows, cols = (int(v) for v in kc["name"].split("_os1_")[1].split("_")[:2])
+    span = kc["Mb"] + (kc["N"] + 2) * rows + (kc["Kb"] + 1) * cols
+    assert not _flags(kc) & MATRIX or span * 2 * int(cfg.fp) < 1 << 31
+    assert (_flags(kc) & MATRIX != 0) == (desc not in ("scfo1.509x509x509", "dcfo2048x2048x47"))
+
+
+def test_matrix_sums_with_64_bit_offsets_stay_refused():
+    cfg = bb.parse_fft_descriptor("scfo2097152.67")
+    tun = dict(factorization=[67], Nt=16, Mb=16, Kb=1, no_pad=True)
+    assert bb.kernel_configuration(cfg, tuning=dict(tun, flags=PER_TILE_IDS))["Mb"] == 16
+    with pytest.raises(bb.BadConfiguration):
+        bb.kernel_configuration(cfg, tuning=dict(tun, flags=PER_TILE_IDS | MATRIX))
+
+
+@pytest.mark.parametrize("t,d", [(0, -1), (1, -1), (2, 1)])
+@pytest.mark.parametrize("N", [41, 67, 134])
+def test_large_prime_factors_with_64_bit_offsets(N, t, d):
+    """K-columns 2^27 elements apart (the buffers' pages in between are never touched)."""
+    M, K, far, H = 2, 2, 1 << 27, N // 2 + 1
+    n_in, n_out = (H if t == 2 else N), (H if t == 1 else N)
+    packed = [1, M, M * n_in] if t == 1 else [1, M, M * n_out]
+    cfg = _cfg(M, N, K, 4, d, t, *((packed, [1, M, far]) if t < 2 else ([1, M, far], packed)))
+    kc = bb.kernel_configuration(cfg)
+    assert not _flags(kc) & MATRIX
+    rng = np.random.default_rng(N)
+    field = rng.uniform(-1, 1, (K, N, M))
+    if t == 2:
+        x = np.zeros(far + M * H, np.complex64)
+        for k in range(K):
+            x[k * far:k * far + M * H] = np.fft.rfft(field[k], axis=0).ravel()
+        y = runner.run(bb, cfg, x, M * N * K).reshape(K, N, M) / N
+        ref = field
+    else:
+        y = runner.run(bb, cfg, field.astype(np.float32).ravel(), far + M * n_out)
+        y = np.stack([y[k * far:k * far + M * n_out].reshape(n_out, M) for k in range(K)])
+        ref = (np.fft.fft if t == 0 else np.fft.rfft)(field, axis=1)
+    assert np.linalg.norm(y - ref) <= 8 * 1.2e-7 * np.log2(N) * np.linalg.norm(ref)
