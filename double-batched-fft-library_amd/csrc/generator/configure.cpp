@@ -496,6 +496,14 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N, c.ostride);
     bool const real = cfg.type != transform_type::c2c;
     std::size_t const eb = 2 * static_cast<std::size_t>(cfg.fp);
+    // Staged tiles are addressed by 32-bit offsets. `Kb` 0: the tile's K-columns are not chosen
+    // yet (at most 256).
+    auto const stageable = [&](std::size_t Kb) {
+        fft1d_configuration t = c;
+        t.Mb = M;
+        t.Kb = Kb ? Kb : 256;
+        return (in || outp) && t.local_offsets();
+    };
     // Adds the flags of a kernel whose packed sides may be staged; `items`: work-items of the
     // launch.
     auto const stage = [&](std::size_t items) {
@@ -555,7 +563,7 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         // each work-group 32 tiles or more (8 x 512 fp64: 32768 K-columns 694 us against 711
         // staged, 8192 182 / 182, 1000 26.4 / 24.6).
         std::size_t const columns = std::size_t(32) * 256 * tuning.groups_per_cu * tuning.Kb;
-        if ((!in && !outp) || tuning_in.unstaged) {
+        if (!stageable(tuning.Kb) || tuning_in.unstaged) {
             tuning.has_flags = tuning.groups_per_cu != 0; // else the default hints
         } else if (columns && kcols >= columns) {
             tuning.flags = fft1d_per_tile_ids;
@@ -608,6 +616,10 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
         bool staged = matrix ? (in || outp) && tuning.Mb == M
                              : (in || outp) && (keep || choose_tiling(c, kcols, info, tuning));
+        if (staged && !stageable(tuning.Kb)) { // never a matrix tiling, whose offsets have 32 bits
+            tuning = untiled;
+            staged = false;
+        }
         if (staged && !matrix && !keep && !(real && whole_m)) {
             // Tiles above half the LDS leave a CU with nothing to overlap a tile's copies, and
             // tiles of all M columns of few K-columns leave CUs idle: M tiles instead (real
@@ -870,7 +882,7 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         if (outp && M * N * K * (4 + eb) > (mfma ? std::size_t(1) << 30 : std::size_t(34) << 20)) {
             unsigned const plain = c.flags;
             c.flags |= fft1d_stage_out | fft1d_xcd_runs;
-            if (c.lds_bytes() > info.local_memory_size) {
+            if (c.lds_bytes() > info.local_memory_size || !c.local_offsets()) {
                 c.flags = plain;
             }
         }
@@ -901,6 +913,9 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             (c.Mb != M || !packed_columns(M, n_out, c.ostride) || c.store_function)) {
             throw bad_configuration("Staged output needs packed columns, one M tile and no store "
                                     "callback");
+        }
+        if (!c.local_offsets()) {
+            throw bad_configuration("Staged tiles need 32-bit tile offsets");
         }
         if (c.lds_bytes() > info.local_memory_size) {
             throw bad_configuration("Work-group exceeds the local memory size");

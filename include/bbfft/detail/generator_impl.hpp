@@ -107,9 +107,9 @@ enum fft1d_flag : unsigned {
     /// not with fft1d_mfma.
     fft1d_prefetch = 64u,
     /// The work-group copies its tile's input (output) through LDS with 16-byte accesses, and
-    /// the stages read (write) the copy. Packed layouts only (Mb = M, K-columns contiguous),
-    /// without a callback on that side; the input side not with MFMA or the load-first tile
-    /// loop.
+    /// the stages read (write) the copy. Packed sides only (Mb = M, K-columns contiguous), with
+    /// 32-bit offsets within a tile on either side and without a callback on that side; the
+    /// input side not with MFMA or the load-first tile loop.
     fft1d_stage_in = 128u,
     fft1d_stage_out = 256u,
     /// The work-item's index arithmetic and twiddle loads stay inside the tile loop. A launch

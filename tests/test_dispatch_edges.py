@@ -6,7 +6,7 @@ import pytest
 import bbfft_amd as bb
 from emu import runner
 
-PER_TILE_IDS, MATRIX = 512, 2048
+STAGE_IN, STAGE_OUT, PER_TILE_IDS, MATRIX = 128, 256, 512, 2048
 
 
 def _cfg(M, N, K, fp, d, t, istride=None, ostride=None):
@@ -91,3 +91,41 @@ def test_large_prime_factors_with_64_bit_offsets(N, t, d):
         y = np.stack([y[k * far:k * far + M * n_out].reshape(n_out, M) for k in range(K)])
         ref = (np.fft.fft if t == 0 else np.fft.rfft)(field, axis=1)
     assert np.linalg.norm(y - ref) <= 8 * 1.2e-7 * np.log2(N) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+@pytest.mark.parametrize("t,d", [(0, -1), (0, 1), (1, -1), (2, 1)])
+@pytest.mark.parametrize("M,N,K,far", [(1, 16, 32, 1 << 24), (3, 35, 4, 1 << 26),
+                                       (8, 64, 2, 1 << 27)])
+def test_packed_side_beside_64_bit_offsets(M, N, K, far, t, d, fp):
+    """One side packed, the K-columns of the other so far apart that a tile needs 64-bit
+    offsets (shapes of the estimate and of the tuning table): no side is staged, and the kernel
+    computes what the packed layout's does."""
+    H = N // 2 + 1
+    n_in, n_out = M * (H if t == 2 else N), M * (H if t == 1 else N)
+    rng = np.random.default_rng(M)
+    x = rng.uniform(-1, 1, (K, n_in, 1 if t == 1 else 2))
+    x = (x[..., 0] if t == 1 else x[..., 0] + 1j * x[..., 1])
+    npr, npc = (np.float32, np.complex64) if fp == 4 else (np.float64, np.complex128)
+    x = x.astype(npr if t == 1 else npc)
+    packed = _cfg(M, N, K, fp, d, t)
+    tun = bb.kernel_configuration(packed)
+    tun = dict(factorization=tun["factorization"], Nt=tun["Nt"], Mb=M, Kb=1, flags=0)
+    ref = runner.run(bb, packed, x.ravel(), K * n_out, tuning=tun)
+    cfg = _cfg(M, N, K, fp, d, t, ostride=[1, M, far])
+    assert not _flags(bb.kernel_configuration(cfg)) & (STAGE_IN | STAGE_OUT)
+    y = runner.run(bb, cfg, x.ravel(), (K - 1) * far + n_out)
+    y = np.concatenate([y[k * far:k * far + n_out] for k in range(K)])
+    assert np.linalg.norm(y - ref) <= 4 * np.finfo(npr).eps * np.log2(N) * np.linalg.norm(ref)
+    cfg = _cfg(M, N, K, fp, d, t, istride=[1, M, far])
+    assert not _flags(bb.kernel_configuration(cfg)) & (STAGE_IN | STAGE_OUT)
+    assert bb.compile_kernel(cfg) > 1000
+    for flag, st in ((STAGE_OUT, dict(istride=[1, M, far])), (STAGE_IN, dict(ostride=[1, M, far]))):
+        with pytest.raises(bb.BadConfiguration):  # asked for, it is refused
+            bb.kernel_configuration(_cfg(M, N, K, fp, d, t, **st),
+                                    tuning=dict(tun, flags=flag, Kb=(1 << 28) // far))
+
+
+def test_half_input_output_beside_64_bit_offsets():
+    cfg = _cfg(4, 512, 40000, 4, -1, 0, istride=[1, 4, 1 << 28])
+    assert not _flags(bb.half_input_kernel_configuration(cfg, "f16", False)) & STAGE_OUT
