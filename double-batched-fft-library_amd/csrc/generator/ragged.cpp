@@ -26,9 +26,12 @@ namespace {
 
 /// Work-items per work-group of the persistent kernel (at least this many).
 constexpr std::size_t ragged_min_group = 256;
-/// LDS budget of one variant: 160 KB / 6, so that the six work-groups per CU that the occupancy
-/// target (6 waves per SIMD, 4 waves per group) allows also fit in LDS.
-constexpr std::size_t ragged_lds_limit = 26 * 1024;
+/// LDS budget of one variant: 160 KB / 6, so that the six work-groups per CU that an occupancy
+/// target of 6 waves per SIMD (4 waves per group) allows also fit in LDS, and 160 KB / 5 without a
+/// target.
+constexpr std::size_t ragged_lds_limit(unsigned waves_per_eu) {
+    return (waves_per_eu >= 6 ? 26 : 32) * 1024;
+}
 /// Largest radix of a variant. All variants share one kernel, whose register allocation is the
 /// largest of the variants', so one wide radix would lower the occupancy of every job.
 constexpr int ragged_radix_max = 12;
@@ -118,12 +121,8 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
     // BBFFT_RAGGED_GROUP / BBFFT_RAGGED_LDS override the common group size and the LDS budget
     // of a variant (measurements)
     std::size_t G = ragged_min_group;
-    std::size_t lds_limit = ragged_lds_limit;
     if (char const *g = std::getenv("BBFFT_RAGGED_GROUP")) {
         G = std::max<std::size_t>(64, static_cast<std::size_t>(std::atoi(g)));
-    }
-    if (char const *l = std::getenv("BBFFT_RAGGED_LDS")) {
-        lds_limit = static_cast<std::size_t>(std::atoi(l));
     }
     for (std::size_t v = 0; v < keys.size(); ++v) {
         auto const &[N, M, d] = keys[v];
@@ -162,29 +161,50 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
         G = std::max(G, t.Mb * t.Nt);
     }
     G = std::min<std::size_t>(G, std::min<std::size_t>(1024, info.max_work_group_size));
+    // Occupancy target (BBFFT_RAGGED_WAVES overrides it for measurements). Radices above 16 (prime
+    // factors) would spill under it: 128 jobs of 61 points fp32 2.69 ms at 5 waves, 0.52 without a
+    // target.
+    bool const narrow = std::all_of(tune.begin(), tune.end(), [](fft1d_tuning const &t) {
+        return *std::max_element(t.factorization.begin(), t.factorization.end()) <= 16;
+    });
+    rk.waves_per_eu = cfg.fp == precision::f32 && narrow ? 6u : 0u;
+    if (char const *w = std::getenv("BBFFT_RAGGED_WAVES")) {
+        rk.waves_per_eu = static_cast<unsigned>(std::atoi(w));
+    }
+    std::size_t lds_limit = ragged_lds_limit(rk.waves_per_eu);
+    if (char const *l = std::getenv("BBFFT_RAGGED_LDS")) {
+        lds_limit = std::max<std::size_t>(64, static_cast<std::size_t>(std::atoi(l)));
+    }
     // K tile: fill the common work-group, within the LDS budget.
     for (std::size_t v = 0; v < keys.size(); ++v) {
         auto const &[N, M, d] = keys[v];
         fft1d_tuning &t = tune[v];
+        configuration const job = variant_configuration(cfg.fp, M, N, static_cast<direction>(d));
+        t.Kb = 1;
+        std::size_t const lds = configure_fft1d(job, info, t).lds_bytes(); // of one K-column
         t.Kb = std::max<std::size_t>(1, G / (t.Mb * t.Nt));
+        if (lds) {
+            t.Kb = std::max<std::size_t>(1, std::min(t.Kb, lds_limit / lds));
+        }
         if (t.Mb >= M) {
             // The tiles of a job are packed: staged through LDS. 256 jobs of the serving mix (7.4
             // GB in and out) 1.50 ms against 1.70 with per-element accesses; copying the next
             // tile's input ahead into a second buffer halves the work-groups per CU: 1.67.
             // Streamed loads gain 1 % there and lose what a cache holds of smaller batches (64
             // jobs of 512 and 500 points, 0.35 GB: 82 us plain, 94 streamed, 93 per element).
-            t.flags |= fft1d_stage_in | fft1d_stage_out;
-            t.flags &= ~unsigned(fft1d_nontemporal_load);
-        }
-        fft1d_configuration c;
-        for (;;) {
-            c = configure_fft1d(variant_configuration(cfg.fp, M, N, static_cast<direction>(d)),
-                                info, t);
-            if (c.lds_bytes() <= lds_limit || t.Kb == 1) {
-                break;
+            // A single stage needs no LDS of its own, so that its staged tile may have to be
+            // narrower. Down to a third of the work-items that still gains (128 jobs of 17 points
+            // fp64 126 us against 175), with a quarter it loses (31 points fp64 442 / 338).
+            std::size_t const column = M * N * 2 * static_cast<std::size_t>(cfg.fp);
+            std::size_t const fit = (lds_limit - 12) / column;
+            std::size_t const Kb = std::max<std::size_t>(1, std::min(t.Kb, fit));
+            if (Kb * column + 12 <= std::max(lds_limit, lds) && 3 * Kb >= t.Kb) {
+                t.Kb = Kb;
+                t.flags |= fft1d_stage_in | fft1d_stage_out;
+                t.flags &= ~unsigned(fft1d_nontemporal_load);
             }
-            t.Kb = t.Kb / 2;
         }
+        fft1d_configuration const c = configure_fft1d(job, info, t);
         if (c.work_group_size() > G) {
             throw bad_configuration("Ragged variant exceeds the common work-group size");
         }
@@ -197,11 +217,6 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
         rk.variants.push_back(c);
     }
     rk.group_size = G;
-    // occupancy target (BBFFT_RAGGED_WAVES overrides it for measurements)
-    rk.waves_per_eu = cfg.fp == precision::f32 ? 6u : 0u;
-    if (char const *w = std::getenv("BBFFT_RAGGED_WAVES")) {
-        rk.waves_per_eu = static_cast<unsigned>(std::atoi(w));
-    }
     // Table order: grouped by variant (work-groups running at the same time then tend to run
     // the same code), jobs of one variant in their given order.
     rk.order.resize(cfg.jobs.size());

@@ -129,3 +129,35 @@ def test_packed_side_beside_64_bit_offsets(M, N, K, far, t, d, fp):
 def test_half_input_output_beside_64_bit_offsets():
     cfg = _cfg(4, 512, 40000, 4, -1, 0, istride=[1, 4, 1 << 28])
     assert not _flags(bb.half_input_kernel_configuration(cfg, "f16", False)) & STAGE_OUT
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+def test_ragged_batches_take_every_register_length(fp):
+    """One stage of a large prime has a wide K tile and no LDS of its own: its staged tile is
+    made narrower or the variant is not staged, never refused."""
+    from bbfft_amd import ragged
+    for N in (13, 17, 31, 37, 41, 43, 47, 53, 59, 61, 122):
+        for M in (1, 3, 8, 33):
+            jobs = [ragged.Job(M, N, 300, -1, 0, 0)]
+            kc = ragged.kernel_configuration(jobs, fp)
+            vc = ragged.variant_configuration(jobs, 0, fp)
+            assert kc["lds_bytes"] <= 32 * 1024 or vc["Kb"] == 1, (N, M)
+            assert vc["Kb"] * M * vc["Nt"] * 3 > 256 - M * vc["Nt"] or len(vc["factorization"]) > 1
+
+
+@pytest.mark.parametrize("fp", [4, 8])
+def test_ragged_jobs_of_one_prime_stage(fp):
+    """Staged and unstaged single stages in one launch, in place and not."""
+    import oracle
+    from bbfft_amd import ragged
+    jobs = ragged.pack([ragged.Job(1, 17, 70, -1), ragged.Job(4, 31, 9, 1),
+                        ragged.Job(1, 41, 5, -1), ragged.Job(3, 12, 30, 1)])
+    n = ragged.total_elements(jobs)
+    x = oracle.uniform_complex(17, n)
+    for in_place in (False, True):
+        y = runner.run_ragged(ragged, jobs, x.copy(), n, precision=fp, grid=3, in_place=in_place)
+        for j in jobs:
+            st = [1, j.M, j.M * j.N]
+            s = slice(j.in_offset, j.in_offset + j.elements)
+            ref = oracle.fft(1, [j.M, j.N, j.K], st, st, 0, j.direction, x[s])
+            assert oracle.rel_l2(y[s], ref) <= oracle.tolerance(fp, j.N), j
