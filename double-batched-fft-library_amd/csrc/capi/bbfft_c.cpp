@@ -722,42 +722,28 @@ int bbfft_aot_generate_ragged(int prec, const bbfft_ragged_job *jobs, size_t num
                               const char *device_info, const char *arch, const char *out_path) {
     return guarded([&] {
         require(device_info && arch && out_path, "null argument");
-        auto const batch = ragged_of(prec, jobs, num_jobs);
-        auto const info = parse_device_info(device_info);
-        // the kernels of large and of small batches of these variants (fp64: one for all sizes)
-        auto const staged = configure_ragged(batch, info, ragged_tiles::staged);
-        auto const direct = configure_ragged(batch, info, ragged_tiles::direct);
-        std::vector<hip::archive_entry> entries;
-        for (auto const *k : {&staged, &direct}) {
-            if (k == &direct && (batch.fp == precision::f64 ||
-                                 direct.identifier() == staged.identifier())) {
-                continue;
-            }
-            std::ostringstream os;
-            generate_ragged(os, *k);
-            hip::archive_entry e;
-            e.arch = arch;
-            e.kernel_names.push_back(k->identifier());
-            e.code = hip::compile_to_native(os.str(), arch);
-            entries.push_back(std::move(e));
-        }
+        auto rk = configure_ragged(ragged_of(prec, jobs, num_jobs), parse_device_info(device_info));
+        std::ostringstream os;
+        generate_ragged(os, rk);
+        std::vector<hip::archive_entry> entries(2);
+        entries[0].arch = arch;
+        entries[0].kernel_names.push_back(rk.identifier());
+        entries[0].code = hip::compile_to_native(os.str(), arch);
         // The plain kernel of each variant with a K tile of 1 and no access hints (the same
         // arithmetic per job).
-        hip::archive_entry plain;
         std::ostringstream ps;
         std::set<std::string> seen;
-        for (auto const &v : staged.variants) {
+        for (auto const &v : rk.variants) {
             auto p = v;
             p.Kb = 1;
             p.flags = 0;
             if (seen.insert(p.identifier()).second) {
                 generate_fft1d(ps, p);
-                plain.kernel_names.push_back(p.identifier());
+                entries[1].kernel_names.push_back(p.identifier());
             }
         }
-        plain.arch = arch;
-        plain.code = hip::compile_to_native(ps.str(), arch);
-        entries.push_back(std::move(plain));
+        entries[1].arch = arch;
+        entries[1].code = hip::compile_to_native(ps.str(), arch);
         hip::write_archive(out_path, entries);
     });
 }

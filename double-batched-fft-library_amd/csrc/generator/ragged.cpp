@@ -27,8 +27,8 @@ namespace {
 /// Work-items per work-group of the persistent kernel (at least this many).
 constexpr std::size_t ragged_min_group = 256;
 /// LDS budget of one variant: 160 KB / 6, so that the six work-groups per CU that an occupancy
-/// target of 6 waves per SIMD (4 waves per group) allows also fit in LDS, and 160 KB / 5 with
-/// fewer waves or without a target.
+/// target of 6 waves per SIMD (4 waves per group) allows also fit in LDS, and 160 KB / 5 without a
+/// target.
 constexpr std::size_t ragged_lds_limit(unsigned waves_per_eu) {
     return (waves_per_eu >= 6 ? 26 : 32) * 1024;
 }
@@ -81,7 +81,7 @@ std::size_t ragged_kernel_configuration::lds_bytes() const {
 }
 
 ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
-                                             device_info const &info, ragged_tiles kind) {
+                                             device_info const &info) {
     if (cfg.fp != precision::f32 && cfg.fp != precision::f64) {
         throw bad_configuration("Unsupported precision");
     }
@@ -167,38 +167,7 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
     bool const narrow = std::all_of(tune.begin(), tune.end(), [](fft1d_tuning const &t) {
         return *std::max_element(t.factorization.begin(), t.factorization.end()) <= 16;
     });
-    // K tile: fill the common work-group, within the LDS budget.
-    std::vector<std::size_t> lds(keys.size()); // of one K-column
-    auto const tile_columns = [&](std::size_t v, std::size_t limit) {
-        std::size_t const Kb = G / (tune[v].Mb * tune[v].Nt);
-        return std::max<std::size_t>(1, lds[v] ? std::min(Kb, limit / lds[v]) : Kb);
-    };
-    for (std::size_t v = 0; v < keys.size(); ++v) {
-        auto const &[N, M, d] = keys[v];
-        tune[v].Kb = 1;
-        lds[v] = configure_fft1d(variant_configuration(cfg.fp, M, N, static_cast<direction>(d)),
-                                 info, tune[v])
-                     .lds_bytes();
-    }
-    // Few tiles leave each CU with too little else to run during a tile's copies, and with the
-    // registers of five waves per SIMD: 32 fp32 jobs of 96 and 128 points, 2434 tiles, 25.0 us
-    // staged against 22.4, 8593 tiles of 500 and 512 points 49.3 / 48.6, 11390 of 96 and 128 70.5
-    // / 72.6. fp64, whose accesses per element are twice as long, gains from 1892 tiles on (28.3 /
-    // 31.3).
-    bool staged = kind == ragged_tiles::staged;
-    if (kind == ragged_tiles::by_size) {
-        std::uint64_t tiles = 0;
-        for (std::size_t j = 0; j < cfg.jobs.size(); ++j) {
-            std::size_t const v = rk.job_variant[j], Mb = tune[v].Mb;
-            std::size_t const Kb = tile_columns(v, ragged_lds_limit(6));
-            tiles += (cfg.jobs[j].M + Mb - 1) / Mb * ((cfg.jobs[j].K + Kb - 1) / Kb);
-        }
-        staged = cfg.fp == precision::f64 || tiles >= 40 * 256;
-        if (char const *e = std::getenv("BBFFT_RAGGED_STAGE")) { // on | off: measurements, tests
-            staged = std::string(e) == "on";
-        }
-    }
-    rk.waves_per_eu = cfg.fp == precision::f32 && narrow ? (staged ? 6u : 5u) : 0u;
+    rk.waves_per_eu = cfg.fp == precision::f32 && narrow ? 6u : 0u;
     if (char const *w = std::getenv("BBFFT_RAGGED_WAVES")) {
         rk.waves_per_eu = static_cast<unsigned>(std::atoi(w));
     }
@@ -206,12 +175,18 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
     if (char const *l = std::getenv("BBFFT_RAGGED_LDS")) {
         lds_limit = std::max<std::size_t>(64, static_cast<std::size_t>(std::atoi(l)));
     }
+    // K tile: fill the common work-group, within the LDS budget.
     for (std::size_t v = 0; v < keys.size(); ++v) {
         auto const &[N, M, d] = keys[v];
         fft1d_tuning &t = tune[v];
         configuration const job = variant_configuration(cfg.fp, M, N, static_cast<direction>(d));
-        t.Kb = tile_columns(v, lds_limit);
-        if (staged && t.Mb >= M) {
+        t.Kb = 1;
+        std::size_t const lds = configure_fft1d(job, info, t).lds_bytes(); // of one K-column
+        t.Kb = std::max<std::size_t>(1, G / (t.Mb * t.Nt));
+        if (lds) {
+            t.Kb = std::max<std::size_t>(1, std::min(t.Kb, lds_limit / lds));
+        }
+        if (t.Mb >= M) {
             // The tiles of a job are packed: staged through LDS. 256 jobs of the serving mix (7.4
             // GB in and out) 1.50 ms against 1.70 with per-element accesses; copying the next
             // tile's input ahead into a second buffer halves the work-groups per CU: 1.67.
@@ -223,7 +198,7 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
             std::size_t const column = M * N * 2 * static_cast<std::size_t>(cfg.fp);
             std::size_t const fit = (lds_limit - 12) / column;
             std::size_t const Kb = std::max<std::size_t>(1, std::min(t.Kb, fit));
-            if (Kb * column + 12 <= std::max(lds_limit, lds[v]) && 3 * Kb >= t.Kb) {
+            if (Kb * column + 12 <= std::max(lds_limit, lds) && 3 * Kb >= t.Kb) {
                 t.Kb = Kb;
                 t.flags |= fft1d_stage_in | fft1d_stage_out;
                 t.flags &= ~unsigned(fft1d_nontemporal_load);

@@ -270,21 +270,15 @@ struct BBFFT_EXPORT ragged_kernel_configuration {
 
     std::uint64_t total_tiles() const { return tile_begin.empty() ? 0 : tile_begin.back(); }
     /// Kernel symbol name; depends on the variants, the work-group size and the occupancy
-    /// target only, so the compiled module serves any job list with the same variants (fp32: one
-    /// module for small batches and one for the others).
+    /// target only, so the compiled module serves any job list with the same variants.
     std::string identifier() const;
     /// Bytes of LDS (the largest of the variants).
     std::size_t lds_bytes() const;
 };
 
-/// Access of a ragged kernel's tiles: copied through LDS or per element, chosen by the batch's
-/// size by default.
-enum class ragged_tiles { by_size, staged, direct };
-
 /// Configure the persistent kernel for a ragged batch (validates the jobs).
-BBFFT_EXPORT ragged_kernel_configuration
-configure_ragged(ragged_configuration const &cfg, device_info const &info,
-                 ragged_tiles kind = ragged_tiles::by_size);
+BBFFT_EXPORT ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
+                                                          device_info const &info);
 /// Emit the HIP source of the persistent kernel `name(in, out, table, njobs)`.
 BBFFT_EXPORT void generate_ragged(std::ostream &os, ragged_kernel_configuration const &rk,
                                   std::string_view name = {});

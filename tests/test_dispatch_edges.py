@@ -161,70 +161,3 @@ def test_ragged_jobs_of_one_prime_stage(fp):
             s = slice(j.in_offset, j.in_offset + j.elements)
             ref = oracle.fft(1, [j.M, j.N, j.K], st, st, 0, j.direction, x[s])
             assert oracle.rel_l2(y[s], ref) <= oracle.tolerance(fp, j.N), j
-
-
-def _archive_names(path):
-    import ctypes
-    data = open(path, "rb").read()
-    L = bb._capi.load()
-    need = ctypes.c_size_t()
-    assert L.bbfft_aot_archive_kernels(data, len(data), None, 0, ctypes.byref(need)) == 0
-    buf = ctypes.create_string_buffer(need.value)
-    assert L.bbfft_aot_archive_kernels(data, len(data), buf, need.value, ctypes.byref(need)) == 0
-    return {ln.split()[1] for ln in buf.value.decode().splitlines()}
-
-
-@pytest.mark.parametrize("fp", [4, 8])
-def test_ragged_archive_serves_small_and_large_batches(fp, tmp_path):
-    """fp32 batches of few tiles run a kernel without staged tiles; an archive made for any batch
-    of the same variants holds the kernels of both."""
-    from bbfft_amd import ragged
-    def batch(K):
-        return [ragged.Job(2, 96, K, -1, 0, 0), ragged.Job(1, 128, K, 1, 0, 0)]
-    names = {ragged.kernel_configuration(batch(K), fp)["name"] for K in (1, 1000, 10 ** 6)}
-    assert len(names) == (2 if fp == 4 else 1)
-    out = str(tmp_path / "r.bin")
-    ragged.aot_generate(batch(1000), out, fp)
-    assert names <= _archive_names(out)
-    if fp == 4:  # it changes once, at 40 tiles per CU
-        lo, hi = 1, 10 ** 6
-        while hi - lo > 1:
-            mid = (lo + hi) // 2
-            same = ragged.kernel_configuration(batch(mid))["name"] == \
-                ragged.kernel_configuration(batch(1))["name"]
-            lo, hi = (mid, hi) if same else (lo, mid)
-        assert ragged.kernel_configuration(batch(hi))["total_tiles"] >= 40 * 256
-        assert ragged.kernel_configuration(batch(hi))["total_tiles"] <= 40 * 256 + 2
-
-
-@pytest.mark.skipif(not runner.have_tsan(), reason="no ThreadSanitizer runtime")
-def test_staged_ragged_kernel_is_race_free(monkeypatch):
-    from bbfft_amd import ragged
-    monkeypatch.setenv("BBFFT_RAGGED_STAGE", "on")
-    jobs = ragged.pack([ragged.Job(3, 20, 40, -1), ragged.Job(1, 27, 9, 1), ragged.Job(2, 17, 70, -1)])
-    n, grid = ragged.total_elements(jobs), 2
-    kc = ragged.kernel_configuration(jobs, 4)
-    ok, report = runner.race_check(
-        ragged.generate_source(jobs, 4),
-        f'{kc["name"]}((const float2*)in, (float2*)out, table, {len(jobs)}ul)', 8 * n, 8 * n,
-        grid, kc["group_size"], in_place=True, table=ragged.job_table(jobs, 4, grid=grid))
-    assert ok, report[-3000:]
-
-
-@pytest.mark.parametrize("fp", [4, 8])
-def test_staged_and_direct_ragged_kernels_agree(fp, monkeypatch):
-    """The same bits from both kernels of a batch: M-tiled and whole-tile variants, jobs off the
-    16-byte boundary, tiles of less than 16 bytes."""
-    import oracle
-    from bbfft_amd import ragged
-    jobs, off = [], 1
-    for M, N, K, d in [(3, 20, 50, -1), (200, 12, 2, 1), (1, 27, 90, -1), (1, 1, 3, 1), (2, 60, 7, 1)]:
-        jobs.append(ragged.Job(M, N, K, d, off, off + 2))
-        off += M * N * K + 1
-    x = oracle.uniform_complex(11, off + 4)
-    out = []
-    for stage in ("on", "off"):
-        monkeypatch.setenv("BBFFT_RAGGED_STAGE", stage)
-        out.append(runner.run_ragged(ragged, jobs, x, off + 4, precision=fp, grid=3))
-        assert ("BBFFT_LDS_DMA16(" in ragged.generate_source(jobs, fp)) == (stage == "on")
-    assert np.array_equal(*out)
