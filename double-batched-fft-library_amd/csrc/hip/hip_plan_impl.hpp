@@ -138,6 +138,7 @@ class ragged_plan final : public plan_base {
     std::string name_;
     shared_handle<module_handle_t> mod_;
     hipFunction_t fn_ = nullptr;
+    void *buffer_ = nullptr; // split weights, then the job table at table_
     void *table_ = nullptr;
     unsigned long njobs_ = 0;
     unsigned grid_ = 0, block_ = 0;

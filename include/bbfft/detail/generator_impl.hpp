@@ -279,7 +279,9 @@ struct BBFFT_EXPORT ragged_kernel_configuration {
 /// Configure the persistent kernel for a ragged batch (validates the jobs).
 BBFFT_EXPORT ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
                                                           device_info const &info);
-/// Emit the HIP source of the persistent kernel `name(in, out, table, njobs)`.
+/// Emit the HIP source of the persistent kernel `name(in, out, table, njobs)` and of
+/// `name_split(table, njobs, grid)`, which writes the work split of a launch of `grid`
+/// work-groups into the job table (one work-item of its 256-item work-groups per g = 0 .. grid).
 BBFFT_EXPORT void generate_ragged(std::ostream &os, ragged_kernel_configuration const &rk,
                                   std::string_view name = {});
 /**
@@ -293,6 +295,11 @@ BBFFT_EXPORT void generate_ragged(std::ostream &os, ragged_kernel_configuration 
 BBFFT_EXPORT std::vector<std::uint64_t> ragged_job_table(ragged_configuration const &cfg,
                                                          ragged_kernel_configuration const &rk,
                                                          std::size_t grid);
+/// What `name_split` reads: the elements of the tiles before each table position (njobs + 1
+/// doubles) and per tile (njobs doubles), then, from where its `table` points, the tile starts and
+/// job records of the job table (5 njobs + 1 words).
+BBFFT_EXPORT std::vector<std::uint64_t> ragged_split_input(ragged_configuration const &cfg,
+                                                           ragged_kernel_configuration const &rk);
 
 } // namespace bbfft
 

@@ -161,3 +161,33 @@ def test_ragged_jobs_of_one_prime_stage(fp):
             s = slice(j.in_offset, j.in_offset + j.elements)
             ref = oracle.fft(1, [j.M, j.N, j.K], st, st, 0, j.direction, x[s])
             assert oracle.rel_l2(y[s], ref) <= oracle.tolerance(fp, j.N), j
+
+
+@pytest.mark.parametrize("grid", [1, 2, 7, 255, 256, 257, 3000])
+def test_ragged_split_kernel_writes_the_job_table(grid):
+    """The kernel that divides a batch's tiles on the device writes the work split of the host's
+    job table, with fewer, as many and more work-groups than tiles, and nothing beside it."""
+    import ctypes
+    from bbfft_amd import ragged
+    rng = np.random.default_rng(grid)
+    jobs = ragged.pack([ragged.Job(int(rng.integers(1, 4)), int(n), int(k), -1) for n, k in zip(
+        rng.choice([16, 60, 105, 128], 9), np.exp(rng.uniform(0, 8, 9)))])
+    nj = len(jobs)
+    name = ragged.kernel_configuration(jobs)["name"] + "_split"
+    tu = ('#include "hip_emu.hpp"\n' + ragged.generate_source(jobs) + "\n"
+          'extern "C" int emu_split(unsigned long* table, unsigned long n, unsigned long g) {\n'
+          f"  return emu::launch(g / 256 + 1, 256, [&] {{ {name}(table, n, g); }});\n}}\n")
+    fn = runner._build_so(tu).emu_split
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_ulong, ctypes.c_ulong]
+    want = ragged.job_table(jobs, grid=grid)
+    recs = want[nj + 1:5 * nj + 1].reshape(nj, 4)
+    weight = np.empty(nj)
+    for p in range(nj):
+        vc = ragged.variant_configuration(jobs, int(recs[p][3]))
+        weight[p] = vc["Mb"] * vc["Kb"] * vc["N"]
+    cum = np.concatenate([[0.0], np.cumsum(weight * np.diff(want[:nj + 1]))])
+    buf = np.full(2 * nj + 1 + len(want) + 4, 77, np.uint64)
+    buf[:nj + 1], buf[nj + 1:2 * nj + 1] = cum.view(np.uint64), weight.view(np.uint64)
+    buf[2 * nj + 1:7 * nj + 2] = want[:5 * nj + 1]
+    assert fn(buf.ctypes.data + 8 * (2 * nj + 1), nj, grid) == 0
+    assert np.array_equal(buf[2 * nj + 1:-4], want) and (buf[-4:] == 77).all()
