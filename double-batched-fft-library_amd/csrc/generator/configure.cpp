@@ -585,12 +585,15 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         bool const keep = !real && cfg.fp == precision::f32 && !half_in && (M == 2 || M == 3) &&
                           r <= 16 && M * Nt <= 512;
         fft1d_tuning const untiled = tuning;
-        // Large prime factors on the matrix cores. Radices up to 64 also run in registers, which
+        // Large prime factors on the matrix cores (not with half-precision input, whose access
+        // flags have no such kernel: 4 x 37 x 110000 f16 had the tiling of matrix sums without
+        // them, 234 us against 139). Radices up to 64 also run in registers, which
         // stays the faster way for fp32 below 37 (31 x 2 and 31 x 4, 8 columns: equal), for fp64
         // below 31, and for M tiles up to 61 in fp32 and 41 in fp64 (30 columns: 53 x 2 fp32 36 us
         // against 44, 37 x 2 fp64 29 against 35; but 53 x 2 fp64 88 against 38).
         int const large = cfg.fp == precision::f32 ? 37 : 31;
-        bool matrix = static_cast<int>(r) >= large && is_prime(static_cast<unsigned>(r)) &&
+        bool matrix = !half_in && static_cast<int>(r) >= large &&
+                      is_prime(static_cast<unsigned>(r)) &&
                       std::count(f.begin(), f.end(), static_cast<int>(r)) == 1;
         c.factorization = f;
         c.Nt = Nt;

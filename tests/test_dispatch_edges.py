@@ -191,3 +191,14 @@ def test_ragged_split_kernel_writes_the_job_table(grid):
     buf[2 * nj + 1:7 * nj + 2] = want[:5 * nj + 1]
     assert fn(buf.ctypes.data + 8 * (2 * nj + 1), nj, grid) == 0
     assert np.array_equal(buf[2 * nj + 1:-4], want) and (buf[-4:] == 77).all()
+
+
+@pytest.mark.parametrize("desc,Nt,radix", [
+    ("scfo4.37*100000", 1, 37), ("scfo3.61*50000", 1, 61), ("scfo4.74*40000", 2, 37),
+    ("scfo16.122*10000", 2, 61), ("scfo8.509*3000", 32, 509)])
+def test_half_input_of_large_primes_keeps_the_tiling_of_its_kernel(desc, Nt, radix):
+    """Half-precision input has no matrix sums: its work-items per transform are those of the
+    butterflies in registers (one of them per work-item) and of the vector sums."""
+    kc = bb.half_input_kernel_configuration(desc, "f16", False)
+    assert kc["factorization"][0] == radix and not _flags(kc) & MATRIX
+    assert kc["Nt"] == Nt and kc["work_group_size"] <= 512
