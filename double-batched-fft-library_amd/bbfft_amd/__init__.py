@@ -506,6 +506,7 @@ INPUT_F16 = _capi.INPUT_F16
 INPUT_BF16 = _capi.INPUT_BF16
 MFMA = _capi.MFMA
 PREFETCH = _capi.PREFETCH  # software-pipelined tile loop (fft1d flag)
+ACCESS_BY_RULE = _capi.ACCESS_BY_RULE  # tunings: access flags chosen by the library
 
 
 def half_input_flags(storage="f16", mfma=True) -> int:

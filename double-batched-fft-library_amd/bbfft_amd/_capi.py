@@ -108,6 +108,7 @@ INPUT_F16 = 8
 INPUT_BF16 = 16
 MFMA = 32
 PREFETCH = 64
+ACCESS_BY_RULE = 4096
 
 _lib = None
 

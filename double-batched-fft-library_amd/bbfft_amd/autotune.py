@@ -34,10 +34,10 @@ from . import (GFX950_INFO, PREFETCH, BadConfiguration, BbfftError, default_cach
 TABLE_HEADER = ("# Tuned kernel parameters for gfx950 (MI355X), written by "
                 "`python -m bbfft_amd.autotune`.\n"
                 "# precision type N M : factorization Nt Mb Kb lds_pad flags "
-                "[waves_per_eu [groups_per_cu]]"
+                "[waves_per_eu | rule [groups_per_cu]]"
                 "   # GB/s default -> tuned, descriptor\n"
-                "# Compiled in, an entry with flags 0 and no waves_per_eu is the tiling of a "
-                "staged kernel where the layout is packed.\n")
+                "# rule: the library chooses the access flags (streaming, staged tiles) for the "
+                "layout and size; otherwise the flags apply as given.\n")
 
 
 def _divisors(n):

@@ -445,7 +445,8 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     bool const explicit_tuning = !tuning_in.factorization.empty() || tuning_in.Nt ||
                                  tuning_in.Mb || tuning_in.Kb || tuning_in.lds_pad ||
                                  tuning_in.no_pad || tuning_in.has_flags;
-    unsigned const all_flags = (tuning_in.has_flags ? tuning_in.flags : 0u) | variant;
+    unsigned const all_flags =
+        ((tuning_in.has_flags ? tuning_in.flags : 0u) | variant) & ~unsigned(fft1d_access_by_rule);
     bool const half_in = (all_flags & (fft1d_input_f16 | fft1d_input_bf16)) != 0;
     bool const mfma = (all_flags & fft1d_mfma) != 0;
     if (!explicit_tuning && info.type == device_type::gpu && info.max_subgroup_size() == 64) {
@@ -471,9 +472,18 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             char const *nt = std::getenv("BBFFT_CALLBACK_NT");
             if (cfg.callbacks.load_function && tuning.has_flags &&
                 !(nt && std::string(nt) == "off")) {
+                tuning.flags &= ~unsigned(fft1d_access_by_rule);
                 tuning.flags |= fft1d_nontemporal_store;
             }
         }
+    }
+    // Access flags by rule, of a whole tiling; any other entry's or caller's flags apply as given.
+    bool const by_rule = tuning.has_flags && (tuning.flags & fft1d_access_by_rule) &&
+                         !tuning.factorization.empty() && tuning.Nt && tuning.Mb && tuning.Kb;
+    bool const given_flags = tuning.has_flags && !(tuning.flags & fft1d_access_by_rule);
+    if (tuning.flags & fft1d_access_by_rule) {
+        tuning.flags &= half_in ? 0u : unsigned(fft1d_direct_matrix); // a property of the tiling
+        tuning.has_flags = tuning.flags != 0;
     }
 
     fft1d_configuration c = {};
@@ -555,18 +565,17 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
         c.flags = 0;
     };
-    if (tuning.builtin && tuning.Mb >= M && !mfma && !half_in && tuning.flags == 0 &&
-        !tuning.waves_per_eu) {
-        // A whole-tile entry of the compiled-in table without hints is the tiling of a staged
-        // kernel: 8 x 16 c2c fp32 166 us (524288 K-columns) against 192 (load-first loop), 8 x 512
-        // 176 / 183, 8 x 384 c2r 181 / 233. Its persistent grid, if any, is for launches that give
-        // each work-group 32 tiles or more (8 x 512 fp64: 32768 K-columns 694 us against 711
-        // staged, 8192 182 / 182, 1000 26.4 / 24.6).
+    if (by_rule && tuning.Mb >= M && !mfma && !half_in && info.type == device_type::gpu) {
+        // The tiling of a staged kernel, where the layout allows one: 8 x 16 c2c fp32 166 us (524288
+        // K-columns) against 192 (load-first loop), 8 x 512 176 / 183, 8 x 384 c2r 181 / 233. Its
+        // persistent grid, if any, is for launches that give each work-group 32 tiles or more (8 x
+        // 512 fp64: 32768 K-columns 694 us against 711 staged, 8192 182 / 182, 1000 26.4 / 24.6).
         std::size_t const columns = std::size_t(32) * 256 * tuning.groups_per_cu * tuning.Kb;
         if (!stageable(tuning.Kb) || tuning_in.unstaged) {
-            tuning.has_flags = tuning.groups_per_cu != 0; // else the default hints
+            tuning.has_flags = tuning.flags || tuning.groups_per_cu; // else the default hints
         } else if (columns && kcols >= columns) {
-            tuning.flags = fft1d_per_tile_ids;
+            tuning.flags |= fft1d_per_tile_ids;
+            tuning.has_flags = true;
         } else {
             tuning.groups_per_cu = 0;
             stage(work_items(M, tuning, kcols));
@@ -871,7 +880,8 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         default_hints = fft1d_nontemporal_load | fft1d_nontemporal_store;
     }
     c.flags = (tuning.has_flags ? tuning.flags : default_hints) | variant;
-    if (half_in && !explicit_tuning && info.type == device_type::gpu && c.Mb == M) {
+    if (half_in && !given_flags && (!explicit_tuning || by_rule) &&
+        info.type == device_type::gpu && c.Mb == M) {
         // Half-precision input: four bytes per element leave the loads cheap and their lines
         // shared by neighbouring accesses, so they go through the caches, element by element; the
         // output is staged beyond the 32 MB of L2 (on the matrix cores, whose tiles take more of a

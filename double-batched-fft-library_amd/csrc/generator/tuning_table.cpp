@@ -70,9 +70,14 @@ std::map<key_t, fft1d_tuning> parse(std::string const &text) {
         while (std::getline(fs, f, 'x')) {
             t.factorization.push_back(std::stoi(f));
         }
-        unsigned waves = 0, groups = 0;
-        if (rhs >> waves) { // optional occupancy target
-            t.waves_per_eu = waves;
+        std::string occupancy;
+        if (rhs >> occupancy) { // optional occupancy target, or access flags by rule
+            if (occupancy == "rule") {
+                t.flags |= fft1d_access_by_rule;
+            } else {
+                t.waves_per_eu = static_cast<unsigned>(std::strtoul(occupancy.c_str(), nullptr, 10));
+            }
+            unsigned groups = 0;
             if (rhs >> groups) { // optional persistent grid
                 t.groups_per_cu = groups;
             }
@@ -100,9 +105,6 @@ std::map<key_t, fft1d_tuning> const &table() {
             tab = parse(ss.str());
         } else {
             tab = parse(builtin_table);
-            for (auto &e : tab) {
-                e.second.builtin = true;
-            }
         }
     });
     return tab;

@@ -123,6 +123,10 @@ enum fft1d_flag : unsigned {
     /// that is an odd prime above 16 (once in the factorisation). Work-groups are whole waves, and
     /// offsets within a tile have 32 bits.
     fft1d_direct_matrix = 2048u,
+    /// Tunings only: the tiling is given, and the library chooses the access flags above
+    /// (streaming, staged tiles, ids per tile, XCD runs) for the layout and the call's size, as it
+    /// does for shapes without a tuning. Needs the whole tiling (factorisation, Nt, Mb, Kb).
+    fft1d_access_by_rule = 4096u,
 };
 
 /// Largest radix a stage computes in registers; a larger (odd) radix runs as a direct DFT stage
@@ -150,8 +154,6 @@ struct BBFFT_EXPORT fft1d_tuning {
     /// Persistent launch: this many work-groups per CU loop over the tiles (0 = one work-group
     /// per tile). Does not change the kernel, only its grid.
     unsigned groups_per_cu = 0;
-    /// Entry of the compiled-in table.
-    bool builtin = false;
     /// Kernels whose tiles cannot be staged by the kernel itself (variants of a ragged kernel):
     /// no staged tiles, and the tiling of kernels without them.
     bool unstaged = false;

@@ -70,8 +70,10 @@ typedef struct bbfft_kernel_config {
  * flags: bit 0 non-temporal global loads, bit 1 non-temporal global stores, BBFFT_PREFETCH
  * (c2c / r2c without callbacks: each work-group loads its next tile's inputs while it transforms
  * the current one; for persistent grids, groups_per_cu > 0); used only when has_flags != 0.
+ * BBFFT_ACCESS_BY_RULE beside a whole tiling: the library chooses the access flags for the layout
+ * and size, as for shapes without a tuning.
  * (No reference counterpart: the reference's tiling is fixed by device_info.) */
-enum { BBFFT_PREFETCH = 64 };
+enum { BBFFT_PREFETCH = 64, BBFFT_ACCESS_BY_RULE = 4096 };
 typedef struct bbfft_tuning {
     int factorization[8];
     int num_factors;

@@ -202,3 +202,68 @@ def test_half_input_of_large_primes_keeps_the_tiling_of_its_kernel(desc, Nt, rad
     kc = bb.half_input_kernel_configuration(desc, "f16", False)
     assert kc["factorization"][0] == radix and not _flags(kc) & MATRIX
     assert kc["Nt"] == Nt and kc["work_group_size"] <= 512
+
+
+_NAMES = """
+import sys
+sys.path.insert(0, sys.argv[1])
+import bbfft_amd as bb
+for d in sys.argv[2:]:
+    desc, _, storage = d.partition("@")
+    print(bb.half_input_kernel_configuration(desc, storage.split("-")[0], "mfma" in storage)["name"]
+          if storage else bb.kernel_configuration(bb.parse_fft_descriptor(desc))["name"])
+"""
+
+
+def _names(descs, env):
+    import os
+    import subprocess
+    import sys
+    pkg = os.path.dirname(os.path.dirname(bb.__file__))
+    r = subprocess.run([sys.executable, "-c", _NAMES, pkg, *descs], capture_output=True, text=True,
+                       env=dict(os.environ, **env), check=True)
+    return r.stdout.split()
+
+
+def test_table_entries_mean_the_same_compiled_in_and_from_a_file(tmp_path):
+    """The compiled-in table read from BBFFT_TUNING_FILE gives the same kernels; a file's own flags
+    apply as given, half-precision input included, and `rule` leaves them to the library."""
+    import os
+    from bbfft_amd import autotune
+    inc = os.path.join(os.path.dirname(os.path.dirname(bb.__file__)), "tuning", "gfx950.inc")
+    rows = [autotune._key(ln) for ln in open(inc) if autotune._key(ln)]
+    descs = []
+    for prec, typ, N, M in rows:
+        base, *storage = typ.split("-")
+        if storage != ["ragged"]:
+            d = f"{'s' if prec == 'f32' else 'd'}{'c' if base == 'c2c' else 'r'}" \
+                f"{'b' if base == 'c2r' else 'f'}o{M}.{N}"
+            descs += [f"{d}*{K}" + ("@" + "-".join(storage) if storage else "")
+                      for K in (3, 3000, 300000)]
+    table = tmp_path / "copy.inc"
+    table.write_text(open(inc).read().split('R"TABLE(', 1)[1].split(')TABLE"', 1)[0])
+    assert _names(descs, {}) == _names(descs, {"BBFFT_TUNING_FILE": str(table)})
+    table.write_text("f32 c2c-f16 512 4 : 32x16 16 4 1 16 67\n"
+                     "f32 c2c 60 8 : 10x6 6 8 4 16 0\n"
+                     "f32 c2c 105 8 : 15x7 7 8 2 16 1 4 2\n"
+                     "f64 c2c 60 8 : 6x5x2 12 8 2 16 0 rule 2\n")
+    half, plain, hints, rule = _names(["scfo4.512*60000@f16", "scfo8.60*30000", "scfo8.105*30000",
+                                       "dcfo8.60*30000"], {"BBFFT_TUNING_FILE": str(table)})
+    assert half.endswith("_g75") and "_Kb1_" in half
+    assert "_g" not in plain and "_f10x6_" in plain
+    assert hints.endswith("_g1_w4")
+    assert int(rule.split("_g")[1]) & (STAGE_IN | STAGE_OUT) == STAGE_IN | STAGE_OUT
+
+
+def test_access_by_rule_is_the_default_access_of_a_tiling():
+    for desc in ["scfo8.256*32768", "scfo8.256*100", "dcfo3.100*40000", "srfo1.512*65536",
+                 "scfo8.509*8192", "srbo5.315*9000"]:
+        cfg = bb.parse_fft_descriptor(desc)
+        kc = bb.kernel_configuration(cfg)
+        tun = dict(factorization=kc["factorization"], Nt=kc["Nt"], Mb=kc["Mb"], Kb=kc["Kb"],
+                   lds_pad=kc["lds_pad"], no_pad=kc["lds_pad"] == 0,
+                   flags=bb.ACCESS_BY_RULE | (_flags(kc) & MATRIX))
+        assert bb.kernel_configuration(cfg, tuning=tun)["name"] == kc["name"], desc
+    # an incomplete tiling or one of M tiles has no rule: the hints of a shape without staging
+    cfg = bb.parse_fft_descriptor("scfo8.256*32768")
+    assert _flags(bb.kernel_configuration(cfg, tuning=dict(flags=bb.ACCESS_BY_RULE))) == 3
