@@ -449,8 +449,13 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         ((tuning_in.has_flags ? tuning_in.flags : 0u) | variant) & ~unsigned(fft1d_access_by_rule);
     bool const half_in = (all_flags & (fft1d_input_f16 | fft1d_input_bf16)) != 0;
     bool const mfma = (all_flags & fft1d_mfma) != 0;
+    std::size_t const half = N / 2 + 1;
+    bool const in = packed_columns(M, cfg.type == transform_type::c2r ? half : N,
+                                   {cfg.istride[0], cfg.istride[1], cfg.istride[2]});
+    bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N,
+                                     {cfg.ostride[0], cfg.ostride[1], cfg.ostride[2]});
     if (!explicit_tuning && info.type == device_type::gpu && info.max_subgroup_size() == 64) {
-        gen::lookup_tuning(cfg.fp, cfg.type, N, M, all_flags, tuning);
+        gen::lookup_tuning(cfg.fp, cfg.type, N, M, all_flags, tuning, in || outp);
         if (char const *m = std::getenv("BBFFT_TABLE_FLAGS_CLEAR")) { // A/B: drop entry flags
             tuning.flags &= ~static_cast<unsigned>(std::strtoul(m, nullptr, 0));
         }
@@ -501,9 +506,6 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     std::size_t const kcols = c.K_columns(K);
 
     bool inplace_refused = false;
-    std::size_t const half = N / 2 + 1;
-    bool const in = packed_columns(M, cfg.type == transform_type::c2r ? half : N, c.istride);
-    bool const outp = packed_columns(M, cfg.type == transform_type::r2c ? half : N, c.ostride);
     bool const real = cfg.type != transform_type::c2c;
     std::size_t const eb = 2 * static_cast<std::size_t>(cfg.fp);
     // Staged tiles are addressed by 32-bit offsets. `Kb` 0: the tile's K-columns are not chosen

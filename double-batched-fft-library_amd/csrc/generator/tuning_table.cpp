@@ -1,7 +1,8 @@
 // Persisted autotuning table: per (precision, transform type, N, M) the kernel parameters the
 // autotuner measured fastest on gfx950. The type may carry the input storage of half-input
 // kernels: c2c-f16, c2c-bf16, c2c-f16-mfma, c2c-bf16-mfma; c2c-ragged entries hold the
-// variants of the persistent ragged kernel. Built into the library from tuning/gfx950.inc;
+// variants of the persistent ragged kernel. Built into the library from tuning/gfx950.inc and, for
+// layouts with neither side packed, tuning/gfx950_strided.inc;
 // BBFFT_TUNING_FILE replaces it with a table file of the same format and BBFFT_TUNING=off
 // disables it (heuristics only).
 #include "tuning_table.hpp"
@@ -20,6 +21,10 @@ namespace {
 
 char const builtin_table[] =
 #include "../../tuning/gfx950.inc"
+    ;
+/// Entries of layouts with neither side packed, which have no staged tiles.
+char const builtin_strided_table[] =
+#include "../../tuning/gfx950_strided.inc"
     ;
 
 using key_t = std::tuple<int, int, std::size_t, std::size_t, unsigned>;
@@ -89,8 +94,12 @@ std::map<key_t, fft1d_tuning> parse(std::string const &text) {
     return table;
 }
 
-std::map<key_t, fft1d_tuning> const &table() {
-    static std::map<key_t, fft1d_tuning> tab;
+struct tables {
+    std::map<key_t, fft1d_tuning> all, strided;
+};
+
+tables const &table() {
+    static tables tab;
     static std::once_flag once;
     std::call_once(once, [] {
         char const *off = std::getenv("BBFFT_TUNING");
@@ -98,13 +107,14 @@ std::map<key_t, fft1d_tuning> const &table() {
             return;
         }
         char const *file = std::getenv("BBFFT_TUNING_FILE");
-        if (file && *file) {
+        if (file && *file) { // for every layout
             std::ifstream f(file);
             std::stringstream ss;
             ss << f.rdbuf();
-            tab = parse(ss.str());
+            tab.all = parse(ss.str());
         } else {
-            tab = parse(builtin_table);
+            tab.all = parse(builtin_table);
+            tab.strided = parse(builtin_strided_table);
         }
     });
     return tab;
@@ -113,17 +123,19 @@ std::map<key_t, fft1d_tuning> const &table() {
 } // namespace
 
 bool lookup_tuning(precision fp, transform_type type, std::size_t N, std::size_t M,
-                   unsigned variant, fft1d_tuning &out) {
+                   unsigned variant, fft1d_tuning &out, bool packed) {
     auto const &t = table();
-    auto it = t.find(
-        key_t{static_cast<int>(fp), static_cast<int>(type), N, M, variant & storage_bits});
-    if (it == t.end()) {
-        return false;
+    key_t const key{static_cast<int>(fp), static_cast<int>(type), N, M, variant & storage_bits};
+    for (auto const *m : {&t.strided, &t.all}) {
+        auto const it = m->find(key);
+        if (it != m->end() && (!packed || m == &t.all)) {
+            out = it->second;
+            return true;
+        }
     }
-    out = it->second;
-    return true;
+    return false;
 }
 
-std::size_t tuning_table_size() { return table().size(); }
+std::size_t tuning_table_size() { return table().all.size(); }
 
 } // namespace bbfft::gen

@@ -267,3 +267,30 @@ def test_access_by_rule_is_the_default_access_of_a_tiling():
     # an incomplete tiling or one of M tiles has no rule: the hints of a shape without staging
     cfg = bb.parse_fft_descriptor("scfo8.256*32768")
     assert _flags(bb.kernel_configuration(cfg, tuning=dict(flags=bb.ACCESS_BY_RULE))) == 3
+
+
+def _strided_rows():
+    import os
+    from bbfft_amd import autotune
+    inc = os.path.join(os.path.dirname(os.path.dirname(bb.__file__)), "tuning",
+                       "gfx950_strided.inc")
+    return [ln for ln in open(inc) if autotune._key(ln)]
+
+
+@pytest.mark.parametrize("row", _strided_rows())
+def test_layouts_without_a_packed_side_have_their_own_entries(row):
+    """Padded K-columns, padded rows: the tiling and flags of the row. One packed side: not."""
+    (prec, typ, N, M), rhs = row.split(":")[0].split(), row.split("#")[0].split(":")[1].split()
+    N, M, t = int(N), int(M), {"c2c": 0, "r2c": 1, "c2r": 2}[typ]
+    fac, (Nt, Mb, Kb, pad, flags) = [int(v) for v in rhs[0].split("x")], map(int, rhs[1:6])
+    H = N // 2 + 1
+    ni, no = (H if t == 2 else N), (H if t == 1 else N)
+    for st in ([1, M, M * ni + 1], [1, M, M * no + M]), ([1, M + 2, (M + 2) * ni],
+                                                       [1, M + 1, (M + 1) * no]):
+        kc = bb.kernel_configuration(_cfg(M, N, 5000, 4 if prec == "f32" else 8,
+                                          1 if t == 2 else -1, t, *st))
+        assert (kc["factorization"], kc["Nt"], kc["Mb"], kc["Kb"], kc["lds_pad"], _flags(kc)) == \
+            (fac, Nt, Mb, Kb, pad, flags)
+    kc = bb.kernel_configuration(_cfg(M, N, 5000, 4 if prec == "f32" else 8, 1 if t == 2 else -1, t,
+                                      istride=[1, M, M * ni + M]))
+    assert _flags(kc) & (STAGE_OUT | PER_TILE_IDS)
