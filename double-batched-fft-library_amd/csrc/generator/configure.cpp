@@ -636,15 +636,16 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
         if (staged && !matrix && !keep && !(real && whole_m)) {
             // Tiles above half the LDS leave a CU with nothing to overlap a tile's copies, and
-            // tiles of all M columns of few K-columns leave CUs idle: M tiles instead (real
-            // transforms that run in place keep all M columns).
+            // tiles of all M columns of few K-columns leave CUs idle: the tiles of layouts that
+            // are not packed instead (real transforms that run in place keep all M columns; 36 x
+            // 243 r2c fp32, 4 K-columns, 5.2 us against 6.1 staged).
             fft1d_configuration t = c;
             t.factorization = tuning.factorization;
             t.Kb = tuning.Kb;
             t.lds_pad = tuning.lds_pad;
             t.flags = 0;
             staged = t.lds_bytes() <= info.local_memory_size / 2 &&
-                     (real || M == 1 || kcols >= 256 || M * Nt <= 64);
+                     (real ? kcols >= 64 : M == 1 || kcols >= 256 || M * Nt <= 64);
             if (!staged) {
                 tuning = untiled;
             }
@@ -657,15 +658,18 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         } else if (matrix) {
             tuning.flags |= fft1d_xcd_runs;
             tuning.has_flags = true;
-        } else if (registers && !(real && whole_m)) {
-            // M tiles. Rows of whole 128-byte lines are stored past the caches, 128 to 256 bytes
-            // per tile: 4704 x 80 x 16 fp32 20.0 us (32 columns; 25.1 with 64 columns and hoisted
-            // ids, 21.5 with plain stores). Streamed loads as well: 19.4, but data that the last
-            // kernel left in a cache is lost (512 x 64 x 64 to the spectrum and back 13.2 against
-            // 10.5; 8320 x 128 x 32 from HBM 95.6 against 86.6). Otherwise neighbouring M tiles share the
-            // lines at their seams: the widest tiles, plain accesses and neighbours on one XCD;
-            // 17 x 512 x 2757 fp32 81 us (9 columns) against 323 (6 columns streamed, neighbours
-            // on different XCDs) and 130 (9 columns plain, different XCDs).
+        } else if (registers && !whole_m && !(real && kcols < 64)) {
+            // M tiles, where the default tile does not hold all M columns (where it does, its
+            // streamed accesses are the faster ones: 6 x 363 c2c fp64, padded rows, 206 us against
+            // 225, 16 x 128 fp32 11.9 / 14.3; halved for few K-columns, 5 x 500 fp64 x 209 packed
+            // 9.8 us against 5.8). Rows of whole 128-byte lines are stored past the caches, 128 to
+            // 256 bytes per tile: 4704 x 80 x 16 fp32 20.0 us (32 columns; 25.1 with 64 columns and
+            // hoisted ids, 21.5 with plain stores). Streamed loads as well: 19.4, but data that the
+            // last kernel left in a cache is lost (512 x 64 x 64 to the spectrum and back 13.2
+            // against 10.5; 8320 x 128 x 32 from HBM 95.6 against 86.6). Otherwise neighbouring M
+            // tiles share the lines at their seams: the widest tiles, plain accesses and neighbours
+            // on one XCD; 17 x 512 x 2757 fp32 81 us (9 columns) against 323 (6 columns streamed,
+            // neighbours on different XCDs) and 130 (9 columns plain, different XCDs).
             std::size_t const line = 128 / eb;
             bool const lines = M % line == 0 && c.istride[1] % line == 0 &&
                                c.ostride[1] % line == 0 && c.istride[2] % line == 0 &&

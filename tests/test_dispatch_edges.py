@@ -294,3 +294,19 @@ def test_layouts_without_a_packed_side_have_their_own_entries(row):
     kc = bb.kernel_configuration(_cfg(M, N, 5000, 4 if prec == "f32" else 8, 1 if t == 2 else -1, t,
                                       istride=[1, M, M * ni + M]))
     assert _flags(kc) & (STAGE_OUT | PER_TILE_IDS)
+
+
+@pytest.mark.parametrize("M,N,K,fp,t,pad,Mb", [
+    (6, 363, 6000, 8, 0, 1, 6), (16, 128, 1200, 4, 0, 1, 16), (8, 300, 138, 4, 0, 8, 8),
+    (5, 500, 209, 8, 0, 0, 5), (10, 384, 142, 4, 0, 0, 10), (57, 64, 26, 8, 0, 0, 57),
+    (36, 243, 4, 4, 1, 0, 18), (31, 512, 31, 4, 2, 0, 16)])
+def test_m_tiles_only_where_a_tile_does_not_hold_all_columns(M, N, K, fp, t, pad, Mb):
+    """Layouts without a packed side and few K-columns keep the default tiling and its streamed
+    accesses where that tile holds all M columns; so do real transforms of few K-columns."""
+    H = N // 2 + 1
+    cfg = _cfg(M, N, K, fp, 1 if t == 2 else -1, t, *(
+        ([1, M, M * N + pad], [1, M, M * (H if t == 1 else N) + pad]) if pad else ()))
+    kc = bb.kernel_configuration(cfg)
+    assert kc["Mb"] == Mb and _flags(kc) == 3
+    general = bb.kernel_configuration(cfg, tuning=dict(factorization=kc["factorization"]))
+    assert kc["name"] == general["name"]
