@@ -886,23 +886,36 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         default_hints = fft1d_nontemporal_load | fft1d_nontemporal_store;
     }
     c.flags = (tuning.has_flags ? tuning.flags : default_hints) | variant;
-    if (half_in && !given_flags && (!explicit_tuning || by_rule) &&
+    // Lengths whose sums run in vector code keep streaming small data: 8 x 509 x 258 f16 79 us
+    // against 86 (x 2000 243 / 210).
+    bool const small_sums = direct && M * N * K * (4 + eb) <= std::size_t(34) << 20;
+    if (half_in && !given_flags && (!explicit_tuning || by_rule) && !small_sums &&
         info.type == device_type::gpu && c.Mb == M) {
         // Half-precision input: four bytes per element leave the loads cheap and their lines
-        // shared by neighbouring accesses, so they go through the caches, element by element; the
-        // output is staged beyond the 32 MB of L2 (on the matrix cores, whose tiles take more of a
-        // CU, beyond 1 GB: 4 x 512 x 262144 1050 us against 1097 direct, x 16384 68 / 65, 16 x 384
-        // x 3000 62 / 46). MI355X, vector kernels, streamed loads before: 4 x 512 x 262144 f16
-        // 1086 -> 1026 us, 8 x 64 x 60000 62 -> 54, 16 x 384 x 3000 65 -> 43.
+        // shared by neighbouring accesses, so they go through the caches, element by element.
+        // MI355X, vector kernels, streamed loads before: 8 x 64 x 60000 62 -> 54 us, 16 x 384 x 3000
+        // 65 -> 43. The output is staged beyond the 32 MB of L2 where rows are shorter than 32
+        // bytes (3 x 61 f16 204 us direct, 148 staged). Longer rows gain from 0.9 GB on (4 x 512 x
+        // 32768 130 / 135, x 131072 523 / 512, with two K-columns a tile, a single wave having
+        // nothing to overlap its copies: 531 with one), radices above 32 not at all (16 x 122 491 /
+        // 577); on the matrix cores, whose tiles take more of a CU, long transforms beyond 1 GB (4
+        // x 512 x 40000 163 / 162, x 98304 405 / 390; 2 x 256 x 240000 241 / 248).
         c.flags = variant | fft1d_per_tile_ids;
         if (outp || M * eb >= 24) {
             c.flags |= fft1d_nontemporal_store;
         }
-        if (outp && M * N * K * (4 + eb) > (mfma ? std::size_t(1) << 30 : std::size_t(34) << 20)) {
-            unsigned const plain = c.flags;
+        std::size_t const bytes = M * N * K * (4 + eb);
+        bool const staged = mfma           ? N >= 512 && bytes > std::size_t(1) << 30
+                            : M * eb < 32 ? bytes > std::size_t(34) << 20
+                                           : rmax <= 32 && bytes > std::size_t(900) << 20;
+        if (outp && staged) {
+            fft1d_configuration const plain = c;
             c.flags |= fft1d_stage_out | fft1d_xcd_runs;
+            if (!mfma && c.Mb * c.Nt * c.Kb <= 64) {
+                c.Kb = std::min(2 * c.Kb, kcols);
+            }
             if (c.lds_bytes() > info.local_memory_size || !c.local_offsets()) {
-                c.flags = plain;
+                c = plain;
             }
         }
     }

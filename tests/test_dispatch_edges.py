@@ -310,3 +310,14 @@ def test_m_tiles_only_where_a_tile_does_not_hold_all_columns(M, N, K, fp, t, pad
     assert kc["Mb"] == Mb and _flags(kc) == 3
     general = bb.kernel_configuration(cfg, tuning=dict(factorization=kc["factorization"]))
     assert kc["name"] == general["name"]
+
+
+def test_half_input_stages_long_rows_of_large_data_only():
+    """Output rows of 32 bytes and more are staged from 0.9 GB on (radices to 32), with two
+    K-columns a tile where one is a single wave; shorter rows beyond the L2."""
+    def conf(desc):
+        kc = bb.half_input_kernel_configuration(desc, "f16", False)
+        return bool(_flags(kc) & STAGE_OUT), kc["Kb"]
+    assert conf("scfo4.512*16384") == (False, 1) and conf("scfo4.512*65536") == (True, 2)
+    assert conf("scfo16.122*60000")[0] is False and conf("scfo3.61*50000")[0] is True
+    assert conf("scfo3.61*2000")[0] is False
