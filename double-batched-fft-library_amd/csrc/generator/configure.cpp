@@ -353,12 +353,23 @@ bool choose_tiling(fft1d_configuration c, std::size_t kcols, device_info const &
     std::size_t const wg_max = std::min<std::size_t>(1024, info.max_work_group_size);
     double const real = c.type != transform_type::c2c ? 1.0 : 0.0;
     double const words = c.fp == precision::f32 ? 2.0 : 4.0; // registers of a complex value
+    c.lds_pad = n >= 32 && (stages > 1 || real > 0.0) ? 16 : 0;
+    // Stages beyond the fewest. A stage more is a rounding more, which fp64 results show (96 c2c
+    // 1.63e-16 against 1.53e-16, 384 c2c 2.01e-16 / 1.97e-16, 12 r2c 1.38e-16 / 1.22e-16) and which
+    // only some shapes are faster for (c2c 96 to 300: 0.9 to 1.03 of the time; 384 and 500 with four
+    // stages 1.02 to 1.1; r2c and c2r of 256 to 512 with three 0.8 to 0.95). Half-precision input,
+    // whose tiles are read element by element, pays for it (1 x 100 x 10000 f16 6.1 us against 5.0).
+    bool const half_in = (c.flags & (fft1d_input_f16 | fft1d_input_bf16)) != 0;
+    if (c.fp == precision::f32 && !half_in) {
+        ++stages;
+    } else if (stages == 1 ? n >= 8 : stages == 2 && !half_in && (real > 0.0 || n >= 256)) {
+        ++stages;
+    }
     bool found = false;
     double best = 0.0;
     c.Mb = M;
-    c.lds_pad = n >= 32 && (stages > 1 || real > 0.0) ? 16 : 0;
     for (auto const &f : facs) {
-        if (f.size() > stages + 1) {
+        if (f.size() > stages) {
             continue;
         }
         c.factorization = f;

@@ -321,3 +321,11 @@ def test_half_input_stages_long_rows_of_large_data_only():
     assert conf("scfo4.512*16384") == (False, 1) and conf("scfo4.512*65536") == (True, 2)
     assert conf("scfo16.122*60000")[0] is False and conf("scfo3.61*50000")[0] is True
     assert conf("scfo3.61*2000")[0] is False
+
+
+@pytest.mark.parametrize("desc,stages", [("dcfo3.96*70000", 2), ("dcfo3.100*3000", 2),
+                                         ("dcfo1.384*40000", 3), ("dcfo5.500*3000", 3),
+                                         ("drfo3.500*3000", 3)])
+def test_fp64_transforms_take_no_stage_for_a_rounding(desc, stages):
+    """c2c of two stages and any length of three keep the fewest stages in double precision."""
+    assert len(bb.kernel_configuration(bb.parse_fft_descriptor(desc))["factorization"]) == stages
