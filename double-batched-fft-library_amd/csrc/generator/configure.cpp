@@ -567,6 +567,9 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         if (!c.store_function && (outp || M * eb >= 24) && filled) {
             tuning.flags |= (outp ? fft1d_stage_out : 0u) | fft1d_nontemporal_store;
         }
+        if (!filled && r <= 32 && M * eb >= 24) { // 15 x 58 x 1607 c2c fp64 12.3 us, plain 14.9
+            tuning.flags |= fft1d_nontemporal_load | fft1d_nontemporal_store;
+        }
         tuning.has_flags = true;
         c.Mb = M;
         c.Kb = tuning.Kb;
@@ -641,7 +644,14 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         }
         bool staged = matrix ? (in || outp) && tuning.Mb == M
                              : (in || outp) && (keep || choose_tiling(c, kcols, info, tuning));
-        if (staged && !stageable(tuning.Kb)) { // never a matrix tiling, whose offsets have 32 bits
+        // Tiles of 36 KB and more leave a CU four groups, too few to overlap the copies of one with
+        // the stages of the others: c2c whose default tile holds all M columns keeps that tile and
+        // its streamed accesses. fp64, 256 MB / 64 MB in and out, staged against that: 9 x 256 50.0 /
+        // 16.0 us, 46.9 / 14.5; 12 x 220 57.0 / 19.0, 51.0 / 15.5; 14 x 243 70.2 / 21.2, 58.5 /
+        // 17.8; fp32 48 x 128 49.8 / 15.4, 47.1 / 12.5. (Default M tiles lose to staged tiles of any
+        // size: 12 x 384 fp64 108 us, staged 66.)
+        bool const large_tile = !real && !half_in && whole_m && M * N * eb >= 36000;
+        if (staged && !matrix && (large_tile || !stageable(tuning.Kb))) {
             tuning = untiled;
             staged = false;
         }

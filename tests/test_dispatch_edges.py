@@ -329,3 +329,14 @@ def test_half_input_stages_long_rows_of_large_data_only():
 def test_fp64_transforms_take_no_stage_for_a_rounding(desc, stages):
     """c2c of two stages and any length of three keep the fewest stages in double precision."""
     assert len(bb.kernel_configuration(bb.parse_fft_descriptor(desc))["factorization"]) == stages
+
+
+@pytest.mark.parametrize("M,N,fp,staged", [(9, 256, 8, False), (14, 243, 8, False),
+                                           (48, 128, 4, False), (8, 256, 8, True),
+                                           (12, 384, 8, True), (20, 315, 4, True)])
+def test_large_c2c_tiles_keep_streamed_accesses(M, N, fp, staged):
+    """Tiles of 36 KB and more are staged only where the default tile splits the columns."""
+    kc = bb.kernel_configuration(_cfg(M, N, (1 << 28) // (M * N * 16), fp, -1, 0))
+    assert bool(_flags(kc) & STAGE_IN) == staged
+    if not staged:
+        assert kc["Mb"] == M and _flags(kc) == 3
