@@ -674,12 +674,16 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         if (matrix) {
             tuning.flags = fft1d_per_tile_ids | fft1d_direct_matrix;
         }
+        // rows of whole 64-byte segments on both sides
+        std::size_t const seg = 64 / static_cast<std::size_t>(cfg.fp);
+        bool const aligned = M % seg == 0 && c.istride[1] % seg == 0 && c.ostride[1] % seg == 0 &&
+                             c.istride[2] % seg == 0 && c.ostride[2] % seg == 0;
         if (staged) {
             stage(keep ? M * Nt * kcols : work_items(M, tuning, kcols));
         } else if (matrix) {
             tuning.flags |= fft1d_xcd_runs;
             tuning.has_flags = true;
-        } else if (registers && !whole_m && !(real && kcols < 64)) {
+        } else if (registers && !whole_m && !(real && (aligned || kcols * ((M + 63) / 64) < 64))) {
             // M tiles, where the default tile does not hold all M columns (where it does, its
             // streamed accesses are the faster ones: 6 x 363 c2c fp64, padded rows, 206 us against
             // 225, 16 x 128 fp32 11.9 / 14.3; halved for few K-columns, 5 x 500 fp64 x 209 packed
@@ -701,10 +705,15 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             if (lines) {
                 mb = std::max(line, std::min(2 * line, 512 / Nt));
             }
-            // few K-columns: smaller tiles until every CU has a work-group or a tile is one wave
-            std::size_t const few = std::max<std::size_t>(1, 64 / Nt);
-            while (!real && mb > few && kcols * ((M + mb - 1) / mb) < 256) {
-                mb = std::max(few, mb / 2);
+            // few K-columns: smaller tiles, of whole 64-byte segments where rows consist of them,
+            // until every CU has a work-group or a tile is one wave
+            std::size_t const few = std::max<std::size_t>(1, 64 / Nt), part = 64 / eb;
+            std::size_t const parts = (256 + kcols - 1) / kcols;
+            if (!real && kcols * ((M + mb - 1) / mb) < 256) {
+                mb = std::min(mb, std::max(few, (M + parts - 1) / parts));
+                if (M % part == 0 && mb > part) {
+                    mb -= mb % part;
+                }
             }
             std::size_t mg = (M + mb - 1) / mb;
             c.factorization = f;
