@@ -506,6 +506,9 @@ INPUT_F16 = _capi.INPUT_F16
 INPUT_BF16 = _capi.INPUT_BF16
 MFMA = _capi.MFMA
 PREFETCH = _capi.PREFETCH  # software-pipelined tile loop (fft1d flag)
+STAGE_IN, STAGE_OUT = _capi.STAGE_IN, _capi.STAGE_OUT  # tiles copied through LDS (fft1d flags)
+PER_TILE_IDS = _capi.PER_TILE_IDS  # index arithmetic inside the tile loop
+DIRECT_MATRIX = _capi.DIRECT_MATRIX  # sums of a large prime radix on the matrix cores
 ACCESS_BY_RULE = _capi.ACCESS_BY_RULE  # tunings: access flags chosen by the library
 
 

@@ -108,6 +108,8 @@ INPUT_F16 = 8
 INPUT_BF16 = 16
 MFMA = 32
 PREFETCH = 64
+STAGE_IN, STAGE_OUT, PER_TILE_IDS = 128, 256, 512
+DIRECT_MATRIX = 2048
 ACCESS_BY_RULE = 4096
 
 _lib = None

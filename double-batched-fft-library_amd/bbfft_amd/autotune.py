@@ -6,12 +6,14 @@ hints for each (precision, transform type, N, M), and writes the table the libra
     python -m bbfft_amd.autotune [-o TABLE] [--rounds 2] DESCRIPTOR...
     python -m bbfft_amd.autotune [-o TABLE] --merge --ragged-serving
 
-Search: coordinate descent from the library's heuristic default, one parameter group at a time
-(factorisation + work-items, K tile, M tile, LDS padding, streaming hints, occupancy target,
-persistent grid with and without the load-first tile loop), keeping the fastest. Every
-candidate's output is compared with the default plan's output on the same input (relative L2
-within the precision's tolerance) before it is timed; the default plan itself is covered by the
-GPU parity suite against the FP64 oracle. Time = best of 3 runs of `reps` launches (HIP events);
+Search: coordinate descent from the tiling of the library's default plan, one parameter group at
+a time (factorisation + work-items, K tile, M tile, LDS padding, access flags, occupancy target,
+persistent grid with and without the load-first tile loop), keeping the fastest. The access flags
+are the library's own for the layout and size (staged tiles where they apply; rows marked `rule`)
+or streaming hints of unstaged kernels, whichever is faster. Every candidate's output is compared
+with the default plan's output on the same input (relative L2 within the precision's tolerance)
+before it is timed; the default plan, whose time the rows quote as the first figure, is covered
+by the GPU parity suite against the FP64 oracle. Time = best of 3 runs of `reps` launches (HIP events);
 shapes under 1 GB of input plus output cycle through several input/output pairs, so every
 launch reads from HBM rather than from the 256 MB last-level cache.
 Confirmation (`--confirm ROUNDS`, default 6): the 4 fastest candidates are re-timed in turn,
@@ -25,11 +27,14 @@ import itertools
 import json
 import math
 import os
+import re
 import sys
 import time
 
-from . import (GFX950_INFO, PREFETCH, BadConfiguration, BbfftError, default_cache,
-               kernel_configuration, make_plan, parse_fft_descriptor)
+from . import (ACCESS_BY_RULE, DIRECT_MATRIX, GFX950_INFO, PER_TILE_IDS, PREFETCH, STAGE_IN,
+               STAGE_OUT, BadConfiguration, BbfftError, default_cache,
+               half_input_kernel_configuration, kernel_configuration, make_half_input_plan,
+               make_plan, parse_fft_descriptor)
 
 TABLE_HEADER = ("# Tuned kernel parameters for gfx950 (MI355X), written by "
                 "`python -m bbfft_amd.autotune`.\n"
@@ -193,6 +198,27 @@ class Tuner:
                 "flags": partial["flags"], "waves_per_eu": partial.get("waves_per_eu", 0),
                 "groups_per_cu": partial.get("groups_per_cu", 0)}
 
+    def storage(self):
+        """Arguments of the half-input entry points for this variant."""
+        return ("f16" if self.variant & 8 else "bf16"), bool(self.variant & 32)
+
+    def default_plan(self):
+        """The plan a program gets without a tuning."""
+        if self.variant:
+            return make_half_input_plan(self.cfg, *self.storage(), cache=self.cache)
+        return make_plan(self.cfg, cache=self.cache)
+
+    def default_tuning(self):
+        """The tiling of that plan, with the library's choice of access flags."""
+        kc = half_input_kernel_configuration(self.cfg, *self.storage()) if self.variant \
+            else kernel_configuration(self.cfg, device_info=GFX950_INFO)
+        g = re.search(r"_g(\d+)", kc["name"])
+        matrix = int(g.group(1)) & DIRECT_MATRIX if g else 0
+        return {"factorization": kc["factorization"], "Nt": kc["Nt"], "Mb": kc["Mb"],
+                "Kb": kc["Kb"], "lds_pad": kc["lds_pad"], "no_pad": kc["lds_pad"] == 0,
+                "flags": ACCESS_BY_RULE | matrix | self.variant, "waves_per_eu": 0,
+                "groups_per_cu": 0}
+
     def factorizations(self):
         if self.variant & 32:  # the MFMA stage is a first radix of 16
             return [[16] + f for f in candidate_factorizations(self.nfft // 16, self.fp)
@@ -201,16 +227,15 @@ class Tuner:
 
     def run(self, rounds=2):
         torch = self.torch
-        # reference output and time of the heuristic default (explicit, table-independent)
-        base = self.full_tuning({"flags": self.variant})
-        plan = make_plan(self.cfg, cache=self.cache, tuning=base)
+        # reference output and time of the plan without a tuning
+        plan = self.default_plan()
         plan.execute(self.x, self.ref)
         torch.cuda.synchronize()
         self.default_ms = self.time_plan(plan)
-        self.results[json.dumps(base, sort_keys=True)] = self.default_ms
-        self.log(desc=self.desc, default=base, ms=round(self.default_ms, 5),
-                 GBps=round(self.bytes / self.default_ms / 1e6, 1))
-        best, best_ms = dict(base), self.default_ms
+        self.log(desc=self.desc, default=plan.launches()[0]["kernel"],
+                 ms=round(self.default_ms, 5), GBps=round(self.bytes / self.default_ms / 1e6, 1))
+        best = self.default_tuning()
+        best_ms = self.evaluate(best)
         kcols = (self.K + 1) // 2 if (self.type != 0 and self.N % 2 == 1) else self.K
         for _ in range(rounds):
             # 1) factorisation and work-items per transform (tile re-derived by the library),
@@ -221,7 +246,8 @@ class Tuner:
                 nt0 = self.nfft // max(f[1:] if self.variant & 32 else f)
                 for nt in sorted({nt0, 2 * nt0}):
                     if nt <= 256:
-                        o = {"factorization": f, "Nt": nt, "flags": best["flags"],
+                        o = {"factorization": f, "Nt": nt,
+                             "flags": best["flags"] & ~DIRECT_MATRIX,
                              "lds_pad": best["lds_pad"], "no_pad": best["no_pad"]}
                         opts += [o, dict(o, Kb=1)]
             best, best_ms = self._try(best, best_ms, opts, complete=True)
@@ -236,16 +262,20 @@ class Tuner:
             # 4) LDS padding
             opts = [dict(best, lds_pad=p, no_pad=p == 0) for p in (0, 8, 16, 32)]
             best, best_ms = self._try(best, best_ms, opts)
-            # 5) streaming hints
-            opts = [dict(best, flags=fl | (best["flags"] & PREFETCH) | self.variant)
+            # 5) access flags: streaming hints, or the library's choice
+            opts = [dict(best, flags=fl | (best["flags"] & (PREFETCH | DIRECT_MATRIX)))
                     for fl in (0, 1, 2, 3)]
+            opts.append(dict(best, flags=ACCESS_BY_RULE | (best["flags"] & DIRECT_MATRIX)))
             best, best_ms = self._try(best, best_ms, opts)
-            # 6) occupancy target of the register allocator
-            opts = [dict(best, waves_per_eu=w) for w in (0, 4, 5, 6, 8)]
+            # 6) occupancy target of the register allocator (a row by rule has none)
+            opts = [] if best["flags"] & ACCESS_BY_RULE else \
+                [dict(best, waves_per_eu=w) for w in (0, 4, 5, 6, 8)]
             best, best_ms = self._try(best, best_ms, opts)
             # 7) persistent grid (work-groups per CU looping over the tiles), with and without
             #    loading the next tile's inputs during the current tile
-            pfs = (0, PREFETCH) if self.type != 2 and not self.variant & 32 else (0,)
+            by_rule = best["flags"] & ACCESS_BY_RULE
+            pfs = (0, PREFETCH) if self.type != 2 and not self.variant & 32 and not by_rule \
+                else (0,)
             opts = [dict(best, groups_per_cu=g, flags=(best["flags"] & ~PREFETCH) | pf)
                     for g in (0, 1, 2, 3, 4, 6, 8, 16) for pf in pfs]
             best, best_ms = self._try(best, best_ms, opts)
@@ -317,11 +347,12 @@ def table_line(cfg, tuning, default_ms, best_ms, nbytes, desc):
     if flags & 32:
         typ += "-mfma"
     fac = "x".join(str(f) for f in tuning["factorization"])
-    waves = tuning.get("waves_per_eu", 0)
+    waves = "rule" if flags & ACCESS_BY_RULE else tuning.get("waves_per_eu", 0)
     groups = tuning.get("groups_per_cu", 0)
     extra = f" {waves} {groups}" if groups else (f" {waves}" if waves else "")
+    kept = DIRECT_MATRIX if flags & ACCESS_BY_RULE else ~(STORAGE_BITS | ACCESS_BY_RULE)
     return (f"{prec} {typ} {cfg.shape[1]} {cfg.shape[0]} : {fac} {tuning['Nt']} {tuning['Mb']} "
-            f"{tuning['Kb']} {tuning['lds_pad']} {flags & (3 | PREFETCH)}{extra}   # "
+            f"{tuning['Kb']} {tuning['lds_pad']} {flags & kept}{extra}   # "
             f"{nbytes / default_ms / 1e6:.0f} -> {nbytes / best_ms / 1e6:.0f} GB/s, {desc}")
 
 
@@ -351,7 +382,8 @@ def merge_table(path, new_lines):
 ROTATE_BELOW_BYTES = 1 << 30  # (input + output) bytes below which timing rotates buffers
 ROTATE_BYTES = 2 << 30  # bytes the rotated pairs span together
 RAGGED_GROUP = 256  # work-items of the persistent ragged kernel's work-group
-RAGGED_WAVES = 5  # its occupancy target (waves per SIMD), shared by all variants
+RAGGED_WAVES = 6  # its occupancy target (waves per SIMD), shared by all variants
+RAGGED_ACCESS = STAGE_IN | STAGE_OUT | PER_TILE_IDS  # its variants' tiles
 
 
 def ragged_candidates(nfft, M, rmax=16, group=RAGGED_GROUP):
@@ -369,7 +401,7 @@ def ragged_candidates(nfft, M, rmax=16, group=RAGGED_GROUP):
 
 def _ragged_tuning(f, nt, M, pad, flags):
     return {"factorization": list(f), "Nt": nt, "Mb": M, "Kb": max(1, RAGGED_GROUP // (M * nt)),
-            "lds_pad": pad, "no_pad": pad == 0, "flags": flags,
+            "lds_pad": pad, "no_pad": pad == 0, "flags": flags | RAGGED_ACCESS,
             "waves_per_eu": RAGGED_WAVES, "groups_per_cu": 0}
 
 
@@ -377,9 +409,9 @@ def tune_ragged_serving(reps=20, confirm_rounds=4, confirm_reps=50, elements=1 <
                         workers=16, verbose=True):
     """Tune the variants (N, M) of the seeded ragged serving workload
     (bbfft_amd.ragged.synthetic_serving_jobs) under the persistent kernel's constraints: each
-    candidate (factorisation with radices <= 16, work-items per transform, LDS padding, access
-    hints) runs as a plain kernel with the ragged kernel's work-group size and occupancy target
-    on `elements` complex elements, so register pressure that would spill in the shared kernel
+    candidate (factorisation with radices <= 16, work-items per transform, LDS padding, streamed
+    stores or not) runs as a plain kernel with the ragged kernel's staged tiles, work-group size
+    and occupancy target on `elements` complex elements, so register pressure that would spill in the shared kernel
     shows as a slow candidate. Direction does not change the cost, so forward and backward share
     an entry. Candidates are compiled in parallel first. Returns the table lines
     ("f32 c2c-ragged N M : ...") ordered by the variants' share of the workload."""
@@ -418,7 +450,7 @@ def tune_ragged_serving(reps=20, confirm_rounds=4, confirm_reps=50, elements=1 <
         for _, k in top:
             t = json.loads(k)
             for pad in (0, 16):
-                for fl in (0, 1, 2, 3):
+                for fl in (0, 2):
                     more.append(_ragged_tuning(t["factorization"], t["Nt"], M, pad, fl))
         with ThreadPoolExecutor(max_workers=workers) as ex:
             list(ex.map(lambda t: _compile_quietly(tuner, t), more))

@@ -498,6 +498,7 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
                          !tuning.factorization.empty() && tuning.Nt && tuning.Mb && tuning.Kb;
     bool const given_flags = tuning.has_flags && !(tuning.flags & fft1d_access_by_rule);
     if (tuning.flags & fft1d_access_by_rule) {
+        variant |= all_flags & (fft1d_input_f16 | fft1d_input_bf16 | fft1d_mfma);
         tuning.flags &= half_in ? 0u : unsigned(fft1d_direct_matrix); // a property of the tiling
         tuning.has_flags = tuning.flags != 0;
     }

@@ -340,3 +340,36 @@ def test_large_c2c_tiles_keep_streamed_accesses(M, N, fp, staged):
     assert bool(_flags(kc) & STAGE_IN) == staged
     if not staged:
         assert kc["Mb"] == M and _flags(kc) == 3
+
+
+def test_m_tiles_split_for_few_k_columns_and_aligned_real_rows():
+    kc = bb.kernel_configuration(_cfg(39, 315, 40, 8, -1, 0, [1, 40, 40 * 315], [1, 40, 40 * 315]))
+    assert kc["Mb"] == 6  # 7 x 40 work-groups
+    kc = bb.kernel_configuration(_cfg(32, 256, 46, 8, -1, 0, [1, 40, 40 * 256], [1, 40, 40 * 256]))
+    assert kc["Mb"] == 4  # 64-byte segments
+    for M, flags in ((32960, 3), (32961, 1536)):
+        kc = bb.kernel_configuration(_cfg(M, 8, 127, 4, 1, 2))
+        assert kc["Mb"] == 64 and _flags(kc) == flags
+
+
+@pytest.mark.parametrize("desc,storage", [("scfo8.256*32768", ""), ("scfo8.509*8192", ""),
+                                          ("dcfo3.100*40000", ""), ("srbo5.315*9000", ""),
+                                          ("scfo4.512*65536", "f16"), ("scfo4.512*65536", "bf16-mfma"),
+                                          ("scfo3.61*50000", "f16")])
+def test_autotuner_starts_from_the_default_plan(desc, storage):
+    """The tuner's first candidate, written as a row, is the kernel of the plan without a tuning;
+    a hint row writes its flags and occupancy as they are."""
+    from bbfft_amd import autotune
+    t = autotune.Tuner.__new__(autotune.Tuner)
+    t.cfg = bb.parse_fft_descriptor(desc)
+    t.variant = bb.half_input_flags(storage.split("-")[0], "mfma" in storage) if storage else 0
+    first = t.default_tuning()
+    want = bb.half_input_kernel_configuration(t.cfg, *t.storage())["name"] if storage else \
+        bb.kernel_configuration(t.cfg)["name"]
+    assert bb.kernel_configuration(t.cfg, tuning=first)["name"].split("_w")[0] == want
+    line = autotune.table_line(t.cfg, first, 1.0, 1.0, 1e9, desc)
+    rhs = line.split("#")[0].split(":")[1].split()
+    assert rhs[6] == "rule" and int(rhs[5]) == (MATRIX if "509" in desc else 0)
+    line = autotune.table_line(t.cfg, dict(first, flags=2 | t.variant, waves_per_eu=5), 1.0, 0.5,
+                               1e9, desc)
+    assert line.split("#")[0].split(":")[1].split()[5:] == ["2", "5"]
