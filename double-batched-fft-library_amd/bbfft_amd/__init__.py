@@ -283,10 +283,12 @@ def aot_generate_shard(descriptors: List[str], out_path: str, shard=0, num_shard
 
 
 def aot_generate(descriptors: List[str], out_dir: str, device_info=GFX950_INFO, arch="gfx950",
-                 jobs=8) -> List[str]:
-    """bbfft-aot-generate: archives out_dir/kernels_<i>.bin built by `jobs` processes."""
+                 jobs=8, any_batch=True) -> List[str]:
+    """bbfft-aot-generate: archives out_dir/kernels_<i>.bin built by `jobs` processes, with
+    any_batch for all batch counts from 64 on."""
     from .aot import generate
-    return generate(descriptors, out_dir, device_info=device_info, arch=arch, jobs=jobs)
+    return generate(descriptors, out_dir, device_info=device_info, arch=arch, jobs=jobs,
+                    any_batch=any_batch)
 
 
 def device_info_query(device=0) -> str:

@@ -1,26 +1,67 @@
 """bbfft-aot-generate: compile the kernels of FFT descriptors ahead of time (no GPU needed).
 
-    python -m bbfft_amd.aot -o OUT_DIR [-d DEVICE_INFO] [-a ARCH] [-j JOBS] DESC... | @FILE
+    python -m bbfft_amd.aot -o OUT_DIR [-d DEVICE_INFO] [-a ARCH] [-j JOBS] [--exact-batch]
+        DESC... | @FILE
+
+A shape has several kernels for small, medium and large batches; unless --exact-batch is given, an
+archive holds those of every batch count from 64 on, whatever count a descriptor names.
 
 Reference: tools/aot/main.cpp:22-60 and tools/aot/args.cpp:17-102. hiprtc compiles one program
 at a time per process, so shards of the kernel list are built by separate processes, each
 writing OUT_DIR/kernels_<shard>.bin; a Cache loads the whole directory.
 """
 import argparse
+import math
 import os
+import re
 import subprocess
 import sys
 
 _PKG_PARENT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+def kernel_names(descriptor, device_info=None):
+    """Names of the kernels a plan of the descriptor launches (and of the passes it fuses)."""
+    from . import (GFX950_INFO, fused_configuration, kernel_configuration, num_passes,
+                   parse_fft_descriptor)
+    info = device_info or GFX950_INFO
+    cfg = parse_fft_descriptor(descriptor)
+    names = [kernel_configuration(cfg, p, info)["name"] for p in range(num_passes(cfg))]
+    fused = fused_configuration(cfg, info) if cfg.dim > 1 else None
+    return names + ([fused["name"]] if fused else [])
+
+
+def batch_descriptors(descriptor, device_info=None, most_bytes=288 << 30):
+    """The descriptor and, for every further kernel that its shape has for batch counts from 64 to
+    what `most_bytes` of input and output hold (eight counts an octave), one with such a count.
+    Descriptors with explicit strides stay alone."""
+    from . import parse_fft_descriptor
+    m = re.fullmatch(r"([a-z]{4}(?:\d+\.)?\d+(?:x\d+)*)(?:\*\d+)?", descriptor)
+    if not m:
+        return [descriptor]
+    cfg = parse_fft_descriptor(m.group(1))
+    one = 4 * int(cfg.fp) * math.prod(cfg.shape[:cfg.dim + 1])
+    out, seen = [descriptor], set(kernel_names(descriptor, device_info))
+    steps = max(0, int(8 * math.log2(max(1, most_bytes // (64 * one))))) + 1
+    for i in range(steps):
+        desc = f"{m.group(1)}*{int(64 * 2 ** (i / 8))}"
+        names = set(kernel_names(desc, device_info))
+        if not names <= seen:
+            out.append(desc)
+            seen |= names
+    return out
+
+
 def generate(descriptors, out_dir, device_info=None, arch="gfx950", jobs=8,
-             ragged_serving=False):
-    """Archives of every kernel the descriptors need; with ragged_serving also the persistent
-    kernel of the seeded mixed serving workload (bbfft_amd.ragged.synthetic_serving_jobs) and
-    its per-variant plain kernels, in OUT_DIR/kernels_ragged_serving.bin."""
+             ragged_serving=False, any_batch=True):
+    """Archives of every kernel the descriptors need, with any_batch for all batch counts from 64 on
+    (batch_descriptors); with ragged_serving also the persistent kernel of the seeded mixed serving
+    workload (bbfft_amd.ragged.synthetic_serving_jobs) and its per-variant plain kernels, in
+    OUT_DIR/kernels_ragged_serving.bin."""
     from . import GFX950_INFO
     device_info = device_info or GFX950_INFO
+    if any_batch:
+        descriptors = [b for d in descriptors for b in batch_descriptors(d, device_info)]
     os.makedirs(out_dir, exist_ok=True)
     for f in os.listdir(out_dir):
         if f.startswith("kernels_") and f.endswith(".bin"):
@@ -101,6 +142,8 @@ def main(argv=None):
     ap.add_argument("--embed", metavar="OUT_CPP",
                     help="write the archives given as arguments (or OUT_DIR/kernels_*.bin) "
                          "into a C++ source to link into an executable")
+    ap.add_argument("--exact-batch", action="store_true",
+                    help="the kernels of the batch counts given alone")
     ap.add_argument("--symbol", default="bbfft_aot_archive", help="array name for --embed")
     ap.add_argument("--ragged-serving", action="store_true",
                     help="compile the ragged kernel of the seeded serving workload to --out-file")
@@ -132,7 +175,7 @@ def main(argv=None):
         n = aot_generate_shard(descs, a.out_file, a.shard, a.num_shards, info, a.arch)
         print(f"shard {a.shard}/{a.num_shards}: {n} kernels -> {a.out_file}", flush=True)
         return 0
-    files = generate(descs, a.out_dir, info, a.arch, a.jobs)
+    files = generate(descs, a.out_dir, info, a.arch, a.jobs, any_batch=not a.exact_batch)
     print(f"{len(files)} archives in {a.out_dir}", flush=True)
     return 0
 

@@ -373,3 +373,23 @@ def test_autotuner_starts_from_the_default_plan(desc, storage):
     line = autotune.table_line(t.cfg, dict(first, flags=2 | t.variant, waves_per_eu=5), 1.0, 0.5,
                                1e9, desc)
     assert line.split("#")[0].split(":")[1].split()[5:] == ["2", "5"]
+
+
+@pytest.mark.parametrize("desc", ["scfo8.256", "srfo8.128", "dcfo3.100", "scfo5.315", "srfo1.512",
+                                  "scfo17.363", "scfo8.509", "drbo8.256", "dcfo32x32",
+                                  "srfo96x96x80"])
+def test_archives_serve_any_batch_count(desc):
+    """The descriptors an archive is made from hold the kernels of every batch count from 64 on,
+    whichever count was named; tested at counts between those that were looked at."""
+    import random
+    from bbfft_amd import aot
+    rng = random.Random(desc)
+    d = aot.batch_descriptors(f"{desc}*{rng.randint(64, 10000)}")
+    held = {n for b in d for n in aot.kernel_names(b)}
+    assert len(d) <= 12 and d == list(dict.fromkeys(d))
+    cfg = bb.parse_fft_descriptor(desc)
+    most = (200 << 30) // (4 * int(cfg.fp) * int(np.prod(cfg.shape[:cfg.dim + 1])))
+    for _ in range(200):
+        K = int(round(np.exp(rng.uniform(np.log(64), np.log(max(65, most))))))
+        assert set(aot.kernel_names(f"{desc}*{K}")) <= held, K
+    assert aot.batch_descriptors(desc + "*5")[0] == desc + "*5"
