@@ -69,7 +69,7 @@ namespace emu {
 inline emu_dim3 blockIdx_, gridDim_, blockDim_;
 inline ucontext_t sched_ctx;
 inline std::vector<ucontext_t> fiber_ctx;
-inline std::vector<int> fiber_state; // 0 runnable, 1 at barrier, 2 done
+inline std::vector<int> fiber_state; // 0 runnable, 1 at barrier, 2 done, 3 waits for its wave
 inline unsigned current = 0;
 inline std::size_t barrier_count = 0;
 #ifdef BBFFT_EMU_TSAN
@@ -193,9 +193,29 @@ template <typename Body> int launch(unsigned grid, unsigned block, Body body) {
                     swapcontext(&sched_ctx, &fiber_ctx[i]);
                 }
             }
+            // waves whose work-items have all arrived at a matrix instruction go on
+            bool went_on = false;
+            for (unsigned w0 = 0; w0 < block; w0 += 64) {
+                unsigned const w1 = w0 + 64 < block ? w0 + 64 : block;
+                unsigned waiting = 0;
+                for (unsigned i = w0; i < w1; ++i) {
+                    waiting += state(i) == 3;
+                }
+                for (unsigned i = w0; i < w1 && waiting == w1 - w0; ++i) {
+                    set_state(i, 0);
+                    went_on = true;
+                }
+            }
+            if (went_on) {
+                continue;
+            }
             for (unsigned i = 0; i < block; ++i) {
                 done += state(i) == 2;
                 at_barrier += state(i) == 1;
+            }
+            if (done + at_barrier != block) {
+                rc = 1; // a wave diverged at a matrix instruction
+                break;
             }
             if (done == block) {
                 break;
@@ -227,27 +247,52 @@ template <typename Body> int launch(unsigned grid, unsigned block, Body body) {
 } // namespace emu
 
 namespace emu {
-inline double mfma16_a[16][64], mfma16_b[16][64];
+
+/// All work-items of a wave meet here: matrix instructions exchange operands between the lanes of
+/// a wave, and order nothing else (no ThreadSanitizer synchronisation, no work-group barrier), so
+/// that a missing barrier around them shows.
+inline void wave_rendezvous() {
+    unsigned const me = cur();
+#ifdef BBFFT_EMU_TSAN
+    __tsan_switch_to_fiber(tsan_sched, __tsan_switch_to_fiber_no_sync);
+#endif
+    set_state(me, 3);
+    swapcontext(&fiber_ctx[me], &sched_ctx);
+}
+
+/// Operands in flight, one word per lane and item (relaxed atomics: no race, no order).
+template <typename T> struct lane_words {
+    T word[16][64][8];
+    void put(unsigned w, unsigned l, unsigned e, T v) {
+        __atomic_store(&word[w][l][e], &v, __ATOMIC_RELAXED);
+    }
+    T get(unsigned w, unsigned l, unsigned e) {
+        T v;
+        __atomic_load(&word[w][l][e], &v, __ATOMIC_RELAXED);
+        return v;
+    }
+};
+inline lane_words<double> mfma16_a, mfma16_b;
 
 /// One v_mfma_{f32,f64}_16x16x4 of a wave: A row / B column = lane % 16, inner index lane / 16;
 /// D item r of lane l = column l % 16, row 4 (l / 16) + r (fp32) or 4 r + l / 16 (fp64). Every
-/// lane of the work-group must call it (two work-group barriers).
+/// lane of the wave must call it.
 template <typename T, typename V4> V4 mfma_16x16x4(T a, T b, V4 c) {
     unsigned const lid = cur(), w = lid / 64u, l = lid % 64u;
-    mfma16_a[w][l] = a;
-    mfma16_b[w][l] = b;
-    __syncthreads();
+    mfma16_a.put(w, l, 0, a);
+    mfma16_b.put(w, l, 0, b);
+    wave_rendezvous();
     V4 d = c;
     for (unsigned r = 0; r < 4; ++r) {
         unsigned const i = sizeof(T) == 4 ? 4u * (l / 16u) + r : 4u * r + l / 16u;
         T s = d[r];
         for (unsigned k = 0; k < 4; ++k) {
-            s += static_cast<T>(mfma16_a[w][i + 16u * k]) *
-                 static_cast<T>(mfma16_b[w][l % 16u + 16u * k]);
+            s += static_cast<T>(mfma16_a.get(w, i + 16u * k, 0)) *
+                 static_cast<T>(mfma16_b.get(w, l % 16u + 16u * k, 0));
         }
         d[r] = s;
     }
-    __syncthreads();
+    wave_rendezvous();
     return d;
 }
 } // namespace emu
@@ -256,30 +301,30 @@ template <typename T, typename V4> V4 mfma_16x16x4(T a, T b, V4 c) {
 
 #if defined(__clang__)
 namespace emu {
-inline float mfma_a[16][64][8];
-inline float mfma_b[16][64][8];
+inline lane_words<float> mfma_a, mfma_b;
 
 /// One v_mfma_f32_32x32x16_{f16,bf16} of a wave: A row / B column = lane % 32, inner index
 /// 8 (lane / 32) + item; D item r of lane l = row 8 (r / 4) + 4 (l / 32) + r % 4, column
-/// l % 32. Every lane of the work-group must call it (two work-group barriers).
+/// l % 32. Every lane of the wave must call it.
 template <typename V8, typename F16> F16 mfma_32x32x16(V8 a, V8 b, F16 c) {
     unsigned const lid = cur(), w = lid / 64u, l = lid % 64u;
-    for (int e = 0; e < 8; ++e) {
-        mfma_a[w][l][e] = static_cast<float>(a[e]);
-        mfma_b[w][l][e] = static_cast<float>(b[e]);
+    for (unsigned e = 0; e < 8; ++e) {
+        mfma_a.put(w, l, e, static_cast<float>(a[e]));
+        mfma_b.put(w, l, e, static_cast<float>(b[e]));
     }
-    __syncthreads();
+    wave_rendezvous();
     F16 d = c;
     unsigned const j = l % 32u;
     for (unsigned r = 0; r < 16; ++r) {
         unsigned const i = 8u * (r / 4u) + 4u * (l / 32u) + r % 4u;
         float s = d[r];
         for (unsigned k = 0; k < 16; ++k) {
-            s += mfma_a[w][i + 32u * (k / 8u)][k % 8u] * mfma_b[w][j + 32u * (k / 8u)][k % 8u];
+            s += mfma_a.get(w, i + 32u * (k / 8u), k % 8u) *
+                 mfma_b.get(w, j + 32u * (k / 8u), k % 8u);
         }
         d[r] = s;
     }
-    __syncthreads();
+    wave_rendezvous();
     return d;
 }
 } // namespace emu

@@ -393,3 +393,47 @@ def test_archives_serve_any_batch_count(desc):
         K = int(round(np.exp(rng.uniform(np.log(64), np.log(max(65, most))))))
         assert set(aot.kernel_names(f"{desc}*{K}")) <= held, K
     assert aot.batch_descriptors(desc + "*5")[0] == desc + "*5"
+
+
+def _race(cfg, tun, K, fp, t, drop=None, grid=2):
+    kc = bb.kernel_configuration(cfg, tuning=tun)
+    src = bb.generate_source(cfg, tuning=tun)
+    if drop is not None:  # a planted mistake: barrier number `drop` of the kernel's tile taken out
+        at = [i for i in range(len(src)) if src.startswith("__syncthreads();", i)][drop]
+        src = src[:at] + src[at + len("__syncthreads();"):]
+    rt, ct = ("float", "float2") if fp == 4 else ("double", "double2")
+    call = (f'{kc["name"]}((const {rt if t == 1 else ct}*)in, ({rt if t == 2 else ct}*)out, '
+            f'{K}ul)')
+    M, N = cfg.shape[:2]
+    H = N // 2 + 1
+    n_in, n_out = M * (H if t == 2 else N) * K, M * (H if t == 1 else N) * K
+    return runner.race_check(src, call, n_in * fp * (1 if t == 1 else 2),
+                             n_out * fp * (1 if t == 2 else 2), grid, kc["work_group_size"])
+
+
+@pytest.mark.skipif(not runner.have_tsan(), reason="no ThreadSanitizer runtime")
+@pytest.mark.parametrize("flags", [PER_TILE_IDS | MATRIX,
+                                   PER_TILE_IDS | MATRIX | STAGE_IN | STAGE_OUT,
+                                   PER_TILE_IDS])  # and the vector sums
+@pytest.mark.parametrize("M,N,K,fp,t,d,fac,Nt,Kb", [
+    (2, 67, 7, 4, 0, -1, [67], 32, 2), (2, 134, 3, 8, 0, 1, [67, 2], 64, 1),
+    (2, 134, 3, 8, 0, 1, [2, 67], 64, 1), (1, 134, 5, 4, 1, -1, [67], 64, 2),
+    (2, 67, 5, 4, 2, 1, [67], 32, 1)])
+def test_direct_stages_are_race_free(M, N, K, fp, t, d, fac, Nt, Kb, flags):
+    """Several waves and tiles per work-group; matrix instructions order nothing but a wave's
+    operands."""
+    tun = dict(factorization=fac, Nt=Nt, Mb=M, Kb=Kb, no_pad=True, flags=flags)
+    ok, report = _race(_cfg(M, N, K, fp, d, t), tun, K, fp, t)
+    assert ok, report[-3000:]
+
+
+@pytest.mark.skipif(not runner.have_tsan(), reason="no ThreadSanitizer runtime")
+@pytest.mark.parametrize("drop", range(4))
+def test_race_check_sees_barriers_around_matrix_sums(drop):
+    """[2, 67]: stage 2's exchange, phase 1's slots, the sums' reads, the tile's end."""
+    cfg = _cfg(2, 134, 5, 4, -1, 0)
+    tun = dict(factorization=[2, 67], Nt=64, Mb=2, Kb=1, no_pad=True,
+               flags=PER_TILE_IDS | MATRIX | STAGE_OUT)
+    assert _race(cfg, tun, 5, 4, 0)[0]
+    ok, report = _race(cfg, tun, 5, 4, 0, drop=drop)
+    assert not ok and "ThreadSanitizer" in report
