@@ -375,7 +375,10 @@ bool choose_tiling(fft1d_configuration c, std::size_t kcols, device_info const &
         c.factorization = f;
         for (std::size_t which = 0; which < std::min<std::size_t>(2, f.size()); ++which) {
             std::size_t const Nt = n / static_cast<std::size_t>(f[which]);
-            if ((which && f[1] == f[0]) || M * Nt > wg_max) {
+            // A wide prime radix spread over as many work-items as the other stage has points leaves
+            // most of them idle (4 x 58 c2c fp32 8.7 us, 6.6 with one butterfly each), which the
+            // estimate, fitted to radices up to 17, sees too little of.
+            if ((which && (f[1] == f[0] || f[0] > 23)) || M * Nt > wg_max) {
                 continue;
             }
             c.Nt = Nt;
@@ -395,6 +398,11 @@ bool choose_tiling(fft1d_configuration c, std::size_t kcols, device_info const &
                 }
                 double const waves = static_cast<double>((wg + 63) / 64);
                 double const regs = 36.0 + words * held;
+                // A group of many waves caps the registers of each: 22 x 205 c2c fp64 (41 x 5) with
+                // 902 work-items spilled, 162 us against 24.
+                if (4.0 * std::floor(512.0 / regs) < waves) {
+                    continue;
+                }
                 double const groups = static_cast<double>((kcols + c.Kb - 1) / c.Kb);
                 double resident = std::floor(info.local_memory_size / double(c.lds_bytes())) * waves;
                 resident = std::min(resident, waves * groups / 256.0);

@@ -437,3 +437,19 @@ def test_race_check_sees_barriers_around_matrix_sums(drop):
     assert _race(cfg, tun, 5, 4, 0)[0]
     ok, report = _race(cfg, tun, 5, 4, 0, drop=drop)
     assert not ok and "ThreadSanitizer" in report
+
+
+@pytest.mark.parametrize("M,N,fp,t", [(22, 205, 8, 0), (23, 82, 8, 0), (21, 410, 8, 2),
+                                      (8, 287, 4, 0), (14, 188, 4, 0), (4, 58, 4, 0),
+                                      (1, 87, 8, 1), (6, 473, 4, 0)])
+def test_wide_prime_radices_keep_one_butterfly_per_work_item(M, N, fp, t):
+    """Prime radices above 23 in registers: as many work-items as the stage has butterflies, in
+    groups whose waves leave each the registers it needs."""
+    for K in (20, 300, 5000):
+        kc = bb.kernel_configuration(_cfg(M, N, K, fp, 1 if t == 2 else -1, t))
+        if _flags(kc) & MATRIX:
+            continue
+        n = N // 2 if t and N % 2 == 0 else N
+        assert kc["Nt"] == n // max(kc["factorization"])
+        waves = -(-kc["work_group_size"] // 64)
+        assert (36 + fp // 2 * max(kc["factorization"])) * -(-waves // 4) <= 512
