@@ -343,9 +343,9 @@ def test_large_c2c_tiles_keep_streamed_accesses(M, N, fp, staged):
 
 
 def test_m_tiles_split_for_few_k_columns_and_aligned_real_rows():
-    kc = bb.kernel_configuration(_cfg(39, 315, 40, 8, -1, 0, [1, 40, 40 * 315], [1, 40, 40 * 315]))
-    assert kc["Mb"] == 6  # 7 x 40 work-groups
-    kc = bb.kernel_configuration(_cfg(32, 256, 46, 8, -1, 0, [1, 40, 40 * 256], [1, 40, 40 * 256]))
+    kc = bb.kernel_configuration(_cfg(39, 315, 20, 8, -1, 0, [1, 40, 40 * 315], [1, 40, 40 * 315]))
+    assert kc["Mb"] == 6  # 7 x 20 work-groups
+    kc = bb.kernel_configuration(_cfg(32, 256, 20, 8, -1, 0, [1, 40, 40 * 256], [1, 40, 40 * 256]))
     assert kc["Mb"] == 4  # 64-byte segments
     for M, flags in ((32960, 3), (32961, 1536)):
         kc = bb.kernel_configuration(_cfg(M, 8, 127, 4, 1, 2))
