@@ -202,7 +202,8 @@ ragged_kernel_configuration configure_ragged(ragged_configuration const &cfg,
             if (Kb * column + 12 <= std::max(lds_limit, lds) && 3 * Kb >= t.Kb) {
                 t.Kb = Kb;
                 t.flags |= fft1d_stage_in | fft1d_stage_out;
-                t.flags &= ~unsigned(fft1d_nontemporal_load);
+                // the copies take the place of the load-first loop of a plain kernel's row
+                t.flags &= ~unsigned(fft1d_nontemporal_load | fft1d_prefetch);
             }
         }
         fft1d_configuration const c = configure_fft1d(job, info, t);

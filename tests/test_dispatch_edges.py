@@ -163,6 +163,29 @@ def test_ragged_jobs_of_one_prime_stage(fp):
             assert oracle.rel_l2(y[s], ref) <= oracle.tolerance(fp, j.N), j
 
 
+def test_ragged_batches_take_every_table_row():
+    """A row may carry the load-first loop, which a staged variant has not: 8 columns of 60 points
+    fp64 are planned and right."""
+    import os
+    import oracle
+    from bbfft_amd import autotune, ragged
+    inc = os.path.join(os.path.dirname(os.path.dirname(bb.__file__)), "tuning", "gfx950.inc")
+    rows = [autotune._key(ln) for ln in open(inc) if autotune._key(ln)]
+    for prec, typ, N, M in rows:
+        if typ in ("c2c", "c2c-ragged") and int(M) < 64:
+            ragged.kernel_configuration([ragged.Job(int(M), int(N), 300, -1, 0, 0)],
+                                        int(prec[1:]) // 8)
+    jobs = ragged.pack([ragged.Job(8, 60, 7, -1), ragged.Job(8, 60, 2, 1)])
+    n = ragged.total_elements(jobs)
+    x = oracle.uniform_complex(60, n)
+    y = runner.run_ragged(ragged, jobs, x.copy(), n, precision=8, grid=3)
+    for j in jobs:
+        st = [1, j.M, j.M * j.N]
+        s = slice(j.in_offset, j.in_offset + j.elements)
+        ref = oracle.fft(1, [j.M, j.N, j.K], st, st, 0, j.direction, x[s])
+        assert oracle.rel_l2(y[s], ref) <= oracle.tolerance(8, j.N), j
+
+
 @pytest.mark.parametrize("grid", [1, 2, 7, 255, 256, 257, 3000])
 def test_ragged_split_kernel_writes_the_job_table(grid):
     """The kernel that divides a batch's tiles on the device writes the work split of the host's
