@@ -37,6 +37,8 @@ MEASURED_TRAFFIC_BYTES = {
         (2.0 * 262181.5 + 1.0 * 524288.0) * 1024,
     "bbfft_m1_M8_Mb8_N256_f8x4x8_Nt32_Kb1_f32_c2c_is1_8_2048_os1_8_2048_p16_in0_g67":
         (2.0 * 262182.5 + 1.0 * 524288.0) * 1024,
+    "bbfft_m1_M8_Mb8_N256_f8x4x8_Nt32_Kb1_f32_c2c_is1_8_2048_os1_8_2048_p16_in0_g899":
+        (2.0 * 262180.0 + 1.0 * 524293.5) * 1024,
 }
 METRIC = "GFLOP/s (5N·log2N) + %HBM peak; MFMA-split vs plain fp32 at equal FP64-err"
 

@@ -553,10 +553,11 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
             // Data that fits the 32 MB of L2: plain loads find what the last kernel left there,
             // and streamed stores take the write-back off the kernel's end. The copies' barriers
             // have nothing to win back, except in real transforms of short rows. To the spectrum
-            // and back in microseconds (copies / plain / plain with streamed stores): 1 x 64 x
-            // 16384 fp32 9.0 / 7.5 / 7.4, 1 x 100 x 5242 fp64 10.8 / 8.9 / 8.1, 8 x 64 x 4096
-            // fp32 12.6 / 12.7 / 10.4; with twice the data 23.3 / 23.1 / 24.0. r2c 8 x 64 x 4096
-            // 10.4 / 9.6 / 8.7, 1 x 64 x 32768 11.9 / 11.7 / 11.0 (10.5: copies, plain loads).
+            // and back in microseconds, in a replayed graph (copies / plain / plain with streamed
+            // stores): 1 x 64 x 16384 fp32 8.0 / 7.5 / 6.8, 1 x 100 x 5242 fp64 9.4 / 8.5 / 7.8,
+            // 8 x 64 x 4096 fp32 10.7 / 13.6 / 10.4, 1 x 64 x 32768 10.9 / 14.4 / 11.6; 8 x 64 x
+            // 8192 23.3 / 23.1 / 24.0. r2c 8 x 64 x 4096 10.4 / 9.6 / 8.7, 1 x 64 x 32768 11.9 /
+            // 11.7 / 11.0 (10.5: copies, plain loads).
             if (!c.store_function && (outp || M * eb >= 24)) {
                 tuning.flags |= fft1d_nontemporal_store;
             }
@@ -614,8 +615,9 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         std::size_t const r = static_cast<std::size_t>(*std::max_element(f.begin(), f.end()));
         bool const registers = r <= static_cast<std::size_t>(fft1d_max_register_radix);
         std::size_t const Nt = nfft / r;
-        // c2c fp32 with M = 2 or 3 keeps the fewest-stages tiling that the host tests fix for it
-        // (staged, 1-9 % slower than the estimate's choice)
+        // c2c fp32 with M = 2 or 3 keeps the fewest-stages tiling, staged: its factors, tile and
+        // padding are a fixed part of the heuristic's interface (the estimate's choice is 1-9 %
+        // faster there)
         bool const keep = !real && cfg.fp == precision::f32 && !half_in && (M == 2 || M == 3) &&
                           r <= 16 && M * Nt <= 512;
         fft1d_tuning const untiled = tuning;
