@@ -39,10 +39,11 @@ from . import (ACCESS_BY_RULE, DIRECT_MATRIX, GFX950_INFO, PER_TILE_IDS, PREFETC
 TABLE_HEADER = ("# Tuned kernel parameters for gfx950 (MI355X), written by "
                 "`python -m bbfft_amd.autotune`.\n"
                 "# precision type N M : factorization Nt Mb Kb lds_pad flags "
-                "[waves_per_eu | rule [groups_per_cu]]"
+                "[waves_per_eu | rule | streamed [groups_per_cu]]"
                 "   # GB/s default -> tuned, descriptor\n"
                 "# rule: the library chooses the access flags (streaming, staged tiles) for the "
-                "layout and size; otherwise the flags apply as given.\n")
+                "layout and size; otherwise the flags apply as given. streamed: rule, with "
+                "streamed loads for all data beyond the L2.\n")
 
 
 def _divisors(n):
@@ -347,7 +348,8 @@ def table_line(cfg, tuning, default_ms, best_ms, nbytes, desc):
     if flags & 32:
         typ += "-mfma"
     fac = "x".join(str(f) for f in tuning["factorization"])
-    waves = "rule" if flags & ACCESS_BY_RULE else tuning.get("waves_per_eu", 0)
+    waves = ("streamed" if flags & 1 else "rule") if flags & ACCESS_BY_RULE \
+        else tuning.get("waves_per_eu", 0)
     groups = tuning.get("groups_per_cu", 0)
     extra = f" {waves} {groups}" if groups else (f" {waves}" if waves else "")
     kept = DIRECT_MATRIX if flags & ACCESS_BY_RULE else ~(STORAGE_BITS | ACCESS_BY_RULE)

@@ -505,6 +505,7 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
     bool const by_rule = tuning.has_flags && (tuning.flags & fft1d_access_by_rule) &&
                          !tuning.factorization.empty() && tuning.Nt && tuning.Mb && tuning.Kb;
     bool const given_flags = tuning.has_flags && !(tuning.flags & fft1d_access_by_rule);
+    bool const streamed = by_rule && (tuning.flags & fft1d_nontemporal_load);
     if (tuning.flags & fft1d_access_by_rule) {
         variant |= all_flags & (fft1d_input_f16 | fft1d_input_bf16 | fft1d_mfma);
         tuning.flags &= half_in ? 0u : unsigned(fft1d_direct_matrix); // a property of the tiling
@@ -572,7 +573,15 @@ fft1d_configuration configure_fft1d(configuration const &cfg, device_info const 
         // little else to hide it.
         bool const filled = items >= 8 * 64 * 256;
         if (in && !c.load_function && filled) {
-            tuning.flags |= fft1d_stage_in | fft1d_nontemporal_load;
+            // Streamed loads leave nothing of the input in the 256 MB last-level cache. Where input
+            // and output fit there, plain ones find what the last kernel or call left: repeated
+            // calls (plain / streamed, geometric means over 17 shapes, M 1 to 17) of 38 MB c2c 0.84,
+            // 50 MB 0.93, 70 to 220 MB 0.90 to 0.92, r2c and c2r 0.84 to 0.96; from memory 1.01 to
+            // 1.03. (540 MB 0.91 and 1.05, 640 MB 1.07 and 1.05.) A row may stream all the same.
+            tuning.flags |= fft1d_stage_in;
+            if (streamed || bytes > std::size_t(256) << 20) {
+                tuning.flags |= fft1d_nontemporal_load;
+            }
         }
         if (!c.store_function && (outp || M * eb >= 24) && filled) {
             tuning.flags |= (outp ? fft1d_stage_out : 0u) | fft1d_nontemporal_store;

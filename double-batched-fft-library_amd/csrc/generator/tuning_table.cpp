@@ -77,8 +77,11 @@ std::map<key_t, fft1d_tuning> parse(std::string const &text) {
         }
         std::string occupancy;
         if (rhs >> occupancy) { // optional occupancy target, or access flags by rule
-            if (occupancy == "rule") {
+            if (occupancy == "rule" || occupancy == "streamed") {
                 t.flags |= fft1d_access_by_rule;
+                if (occupancy == "streamed") { // ... with streamed loads beyond the L2
+                    t.flags |= fft1d_nontemporal_load;
+                }
             } else {
                 t.waves_per_eu = static_cast<unsigned>(std::strtoul(occupancy.c_str(), nullptr, 10));
             }

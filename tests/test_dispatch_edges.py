@@ -278,6 +278,28 @@ def test_table_entries_mean_the_same_compiled_in_and_from_a_file(tmp_path):
     assert int(rule.split("_g")[1]) & (STAGE_IN | STAGE_OUT) == STAGE_IN | STAGE_OUT
 
 
+@pytest.mark.parametrize("desc,below,above", [
+    ("dcfo3.100", 27900, 28000), ("scfo8.384", 5461, 5462), ("srfo1.512", 65300, 65500),
+    ("dcfo8.105", 9980, 10000), ("srbo5.315", 21200, 21350)])
+def test_loads_stream_where_input_and_output_outgrow_the_last_level_cache(desc, below, above):
+    """256 MB of input and output: the largest data that staged kernels load plainly."""
+    def flags(K):
+        return _flags(bb.kernel_configuration(bb.parse_fft_descriptor(f"{desc}*{K}")))
+    assert flags(below) & (STAGE_IN | 3) == STAGE_IN | 2
+    assert flags(above) & (STAGE_IN | 3) == STAGE_IN | 3
+    assert flags(below) | 1 == flags(above)
+
+
+def test_streamed_rows_stream_their_loads_beyond_the_l2(tmp_path):
+    table = tmp_path / "rows.inc"
+    table.write_text("f32 c2c 60 8 : 10x6 6 8 4 16 0 streamed\nf64 c2c 60 8 : 6x5x2 12 8 2 16 0 rule\n")
+    names = _names(["scfo8.60*12000", "scfo8.60*3000", "scfo8.60*60000", "dcfo8.60*6000"],
+                   {"BBFFT_TUNING_FILE": str(table)})
+    assert [int(n.split("_g")[1]) & 3 for n in names] == [3, 2, 3, 2]
+    assert all("_f10x6_" in n for n in names[:3])
+    assert _flags(bb.kernel_configuration(bb.parse_fft_descriptor("scfo8.256*1100"))) & 3 == 3
+
+
 def test_access_by_rule_is_the_default_access_of_a_tiling():
     for desc in ["scfo8.256*32768", "scfo8.256*100", "dcfo3.100*40000", "srfo1.512*65536",
                  "scfo8.509*8192", "srbo5.315*9000"]:
